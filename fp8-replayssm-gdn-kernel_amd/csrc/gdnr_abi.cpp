@@ -557,6 +557,34 @@ int launch_decode(const gdnr::ReplayArgs& r, int act, bool fused, bool gate_f32,
   return gdnr::launch_decode_f16(a, fused, gate_f32, stream);
 }
 
+// The ring kernel (gdnr_ring.hip) takes the rings of 17 to kMaxRing tokens
+// with 16-bit activations that the decode kernel leaves (more than two of its
+// workgroups per compute unit, or V = 256): V = 64 (an even group: a
+// workgroup's four waves hold two heads), 128 or 256, any batch the grid's
+// second dimension holds.
+bool ring_eligible(const gdnr::ReplayArgs& a, int act) {
+  if (act != GDNR_DTYPE_BF16 && act != GDNR_DTYPE_F16) return false;
+  return a.L > gdnr::kStepRing && (a.V == 128 || a.V == 256 || (a.V == 64 && a.G % 2 == 0)) && a.B <= 65535 &&
+         decode_offsets_fit(a, elem_size(act));
+}
+int launch_ring(const gdnr::ReplayArgs& r, int act, bool fused, bool gate_f32, void* stream) {
+  gdnr::StepArgs a = make_step_args(r, elem_size(act), gate_f32 ? 4 : elem_size(act));
+  // Waves per value head (V = 128, an even group): two of 64 rows, so that two
+  // heads share their key head's staging, from three workgroups per compute
+  // unit on (what is resident at once); four of 32 rows below that, where
+  // twice the workgroups fill the chip and a flush is half as long. us per
+  // step with staggered fills, four and two waves: B=24, L=64 11.9 and 14.6;
+  // B=37, L=48 14.7 and 18.6; B=64, L=64 22.0 and 21.7; B=256 73 and 54.
+  const int64_t resident = 3 * (int64_t)gdnr::device_cus();
+  a.nwh = a.V == 256 || a.G % 2 || (a.V == 128 && (int64_t)a.B * a.H * (a.G / 2) <= resident) ? 4 : 2;
+  a.gw = 4 / a.nwh;
+  a.units = a.G / a.gw;  // head groups per key head
+  // flushing sequences first, where the workgroups take more than one round
+  a.seq_major = a.flush && a.B <= gdnr::kRingOrder && (int64_t)a.B * a.H * a.units > resident;
+  if (act == GDNR_DTYPE_BF16) return gdnr::launch_ring_bf16(a, fused, gate_f32, stream);
+  return gdnr::launch_ring_f16(a, fused, gate_f32, stream);
+}
+
 int launch_replay(const gdnr::ReplayArgs& a, int act, int mode, bool gate_f32, void* stream) {
   if (act == GDNR_DTYPE_BF16) return gdnr::launch_replay_bf16(a, mode, gate_f32, stream);
   if (act == GDNR_DTYPE_F16) return gdnr::launch_replay_f16(a, mode, gate_f32, stream);
@@ -754,6 +782,7 @@ int gdnr_replay_fp8(const gdnr_tensor* checkpoint, const gdnr_tensor* checkpoint
     fit_decode(&a);
     return hip_status(launch_decode(a, g.act, false, false, stream));
   }
+  if (ring_eligible(a, g.act)) return hip_status(launch_ring(a, g.act, false, false, stream));
   if (a.L <= gdnr::kStepRing && step_offsets_fit(a, elem_size(g.act))) {
     GDNR_TRY(fit_step(&a, elem_size(g.act)));
     return hip_status(launch_step(a, g.act, false, false, stream));
@@ -968,6 +997,7 @@ int gdnr_prep_replay_fp8(const gdnr_tensor* mixed_qkv, const gdnr_tensor* a, con
     fit_decode(&r);
     return hip_status(launch_decode(r, g.act, true, a->dtype == GDNR_DTYPE_F32, stream));
   }
+  if (ring_eligible(r, g.act)) return hip_status(launch_ring(r, g.act, true, a->dtype == GDNR_DTYPE_F32, stream));
   if (r.L <= gdnr::kStepRing && step_offsets_fit(r, elem_size(g.act))) {
     GDNR_TRY(fit_step(&r, elem_size(g.act)));
     return hip_status(launch_step(r, g.act, true, a->dtype == GDNR_DTYPE_F32, stream));
@@ -1017,13 +1047,16 @@ int gdnr_prep_replay_fp8_slots(const gdnr_tensor* mixed_qkv, const gdnr_tensor* 
   r.o_b = out->strides[0];
   r.o_h = out->strides[1];
   // the decode kernel (16-bit activations, rings of <= 16 tokens, or of
-  // <= 64 with V <= 128; 64-bit slot bases, 32-bit offsets inside a slot),
-  // else the step kernel (rings of <= 16 tokens, tensors under 2 GiB), else
-  // the long-ring kernel (rings of up to 64 tokens, every address in 64 bits)
+  // <= 64 with V <= 128 at small batches), else the ring kernel (16-bit
+  // activations, rings of 17 to 64 tokens; both 64-bit slot bases, 32-bit
+  // offsets inside a slot), else the step kernel (rings of <= 16 tokens,
+  // tensors under 2 GiB), else the long-ring kernel (rings of up to 64
+  // tokens, every address in 64 bits)
   if (decode_eligible(r, g.act) && decode_offsets_fit(r, elem_size(g.act))) {
     fit_decode(&r);
     return hip_status(launch_decode(r, g.act, true, a->dtype == GDNR_DTYPE_F32, stream));
   }
+  if (ring_eligible(r, g.act)) return hip_status(launch_ring(r, g.act, true, a->dtype == GDNR_DTYPE_F32, stream));
   if (r.L <= gdnr::kStepRing && step_offsets_fit(r, elem_size(g.act))) {
     GDNR_TRY(fit_step(&r, elem_size(g.act)));
     return hip_status(launch_step(r, g.act, true, a->dtype == GDNR_DTYPE_F32, stream));

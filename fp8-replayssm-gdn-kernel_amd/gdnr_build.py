@@ -33,15 +33,16 @@ DEVICE_FLAGS = [
 ]
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall", "-Wextra"]
 ACTS = ("bf16", "f16", "f32")  # activation dtypes, one kernel object each (GDNR_ACT = index)
-KERNEL_SOURCES = ("gdnr_kernels", "gdnr_step", "gdnr_decode")  # compiled once per activation dtype
+KERNEL_SOURCES = ("gdnr_kernels", "gdnr_step", "gdnr_decode", "gdnr_ring")  # compiled once per activation dtype
 SINGLE_SOURCES = ("gdnr_rmw", "gdnr_formats", "gdnr_status", "gdnr_probe")  # compiled once (dtypes are template arguments)
 # per-source device flags: the decode kernel's first 13 argument dwords are
 # preloaded into SGPRs at wave launch (gfx950 kernarg preload), and its
 # wave-uniform branches (workgroup role, replay or flush) are left as scalar
 # branches rather than structurised into a chain in which one arm's values
-# stay live across the other
+# stay live across the other; the ring kernel's (replay or flush) too
 SOURCE_FLAGS = {"gdnr_decode": ["-mllvm", "-amdgpu-kernarg-preload-count=13",
-                                "-mllvm", "-structurizecfg-skip-uniform-regions=true"]}
+                                "-mllvm", "-structurizecfg-skip-uniform-regions=true"],
+                "gdnr_ring": ["-mllvm", "-structurizecfg-skip-uniform-regions=true"]}
 
 
 def _run(cmd: list[str], verbose: bool) -> None:
