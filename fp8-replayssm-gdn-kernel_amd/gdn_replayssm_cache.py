@@ -28,6 +28,7 @@ import numpy as np
 import torch
 
 import gdn_replayssm_fp8_kernel as gk
+import gdnr_lib
 
 FP8_DTYPE = torch.float8_e4m3fn
 
@@ -102,17 +103,23 @@ class ReplaySSMCache:
         """One full-contract decode step of the batch: batch entry i is the
         sequence in slot slots[i] (0 = padding; its output is meaningless).
         mixed_qkv [B, 2HK + HV V], a, b [B, HV]; returns out [B, HV, V]."""
-        slots, pos, valid, flush = self.metadata(slots)
+        slots = np.ascontiguousarray(slots, dtype=np.int64)
+        if slots.ndim != 1:
+            raise ValueError("slots must be one-dimensional")
+        host = gdnr_lib.host()
         batch = slots.shape[0]
+        # slot, pos, valid_len (int32) and flush (a byte) of each entry, in one
+        # pinned buffer and one copy
+        packed = torch.empty(13 * batch, dtype=torch.uint8, pin_memory=True)
+        host.slot_metadata(self.fill, slots, self.window, packed.numpy())
         if mixed_qkv.shape[0] != batch:
             raise ValueError(f"mixed_qkv has {mixed_qkv.shape[0]} rows for a batch of {batch}")
-        meta = torch.from_numpy(np.stack([slots, pos, valid, flush.astype(np.int64)]).astype(np.int32))
-        meta = meta.pin_memory().to(self.device, non_blocking=True)
+        packed = packed.to(self.device, non_blocking=True)
+        meta = packed[:12 * batch].view(torch.int32).view(3, batch)
         if q_out is None:
             q_out = torch.empty(batch, self.heads, self.key_dim, dtype=self.dtype, device=self.device)
         result = gk.gdn_prep_replay_fp8(mixed_qkv, a, b, a_log, dt_bias, meta[1], self.payload, self.scale, q_out,
                                         self.k_ring, self.v_ring, self.g_ring, self.beta_ring, meta[2],
-                                        meta[3].bool(), block_v=block_v, out=out, state_indices=meta[0])
-        live = slots != 0
-        self.fill[slots[live]] = np.where(flush, 0, valid)[live]
+                                        packed[12 * batch:], block_v=block_v, out=out, state_indices=meta[0])
+        host.advance(self.fill, slots, self.window)
         return result

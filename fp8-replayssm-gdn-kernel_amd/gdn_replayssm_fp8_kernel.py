@@ -48,18 +48,14 @@ FP8_DTYPE = torch.float8_e4m3fn
 VBLOCK = 32
 
 
-def _require_cuda(**tensors: torch.Tensor | None) -> torch.device:
-    device = None
-    for name, t in tensors.items():
-        if t is None:
-            continue
-        if not isinstance(t, torch.Tensor) or not t.is_cuda:
-            raise ValueError(f"{name} must be a tensor on the GPU")
-        if device is None:
-            device = t.device
-        elif t.device != device:
-            raise ValueError(f"{name} is on {t.device}, expected {device}")
-    return device
+_ENTRY = gdnr_lib.ENTRY_IDS
+_REPLAY, _SPLIT, _PREP = _ENTRY["gdnr_replay_fp8"], _ENTRY["gdnr_replay_fp8_split"], _ENTRY["gdnr_prep_ring"]
+_STEP, _STEP_SLOTS = _ENTRY["gdnr_prep_replay_fp8"], _ENTRY["gdnr_prep_replay_fp8_slots"]
+_RMW, _RMW_PACKED = _ENTRY["gdnr_bf16_step"], _ENTRY["gdnr_bf16_step_packed"]
+
+
+def _as_f32(t: torch.Tensor) -> torch.Tensor:
+    return t if t.dtype == torch.float32 else t.float()
 
 
 def _as_i32(t: torch.Tensor) -> torch.Tensor:
@@ -124,8 +120,10 @@ def quantize_checkpoint(state: torch.Tensor, granularity: str = "vblock", tile_s
     (which synchronises, like the reference's ``.item()``) and reports 0.
     """
     base, code, is_int8 = _format(granularity)
-    device = _require_cuda(state=state)
-    state32 = state if state.dtype == torch.float32 else state.float()
+    host = gdnr_lib.host()
+    host.require(("state",), (state,))
+    device = state.device
+    state32 = _as_f32(state)
     if state32.dim() != 4:
         raise ValueError("state must be [B, HV, V, K]")
     batch, heads, value_dim, key_dim = state32.shape
@@ -135,13 +133,10 @@ def quantize_checkpoint(state: torch.Tensor, granularity: str = "vblock", tile_s
     scale = torch.empty(_scale_shape(base, batch, heads, value_dim, key_dim, tile_size), dtype=torch.float16,
                         device=device)
     saturated = torch.empty(scale.shape, dtype=torch.int32, device=device) if saturation else None
-    with torch.cuda.device(device):
-        if base == "vblock" and tile_size == VBLOCK and not is_int8:
-            gdnr_lib.call("gdnr_quantize_vblock32", [state32, payload, scale, saturated],
-                          stream=gdnr_lib.current_stream(device))
-        else:
-            gdnr_lib.call("gdnr_quantize_checkpoint", [state32, payload, scale, saturated], [code, tile_size],
-                          gdnr_lib.current_stream(device))
+    if base == "vblock" and tile_size == VBLOCK and not is_int8:
+        host.call(_ENTRY["gdnr_quantize_vblock32"], (state32, payload, scale, saturated), (), (), None)
+    else:
+        host.call(_ENTRY["gdnr_quantize_checkpoint"], (state32, payload, scale, saturated), (code, tile_size), (), None)
     fraction = float(saturated.sum().item()) / max(state32.numel(), 1) if saturation else 0.0
     return QuantizedCheckpoint(payload, scale, granularity, tile_size, fraction)
 
@@ -150,15 +145,14 @@ def dequantize_checkpoint(checkpoint: QuantizedCheckpoint) -> torch.Tensor:
     """ref:109-134 for every format: float(payload) * float(scale), the scale
     broadcast over its group."""
     base, code, _ = _format(checkpoint.granularity)
-    device = _require_cuda(payload=checkpoint.payload, scale=checkpoint.scale)
-    out = torch.empty(checkpoint.payload.shape, dtype=torch.float32, device=device)
-    with torch.cuda.device(device):
-        if base == "vblock" and checkpoint.tile_size == VBLOCK and checkpoint.payload.dtype != torch.int8:
-            gdnr_lib.call("gdnr_dequantize_vblock32", [checkpoint.payload, checkpoint.scale, out],
-                          stream=gdnr_lib.current_stream(device))
-        else:
-            gdnr_lib.call("gdnr_dequantize_checkpoint", [checkpoint.payload, checkpoint.scale, out],
-                          [code, checkpoint.tile_size], gdnr_lib.current_stream(device))
+    payload, scale = checkpoint.payload, checkpoint.scale
+    host = gdnr_lib.host()
+    host.require(("payload", "scale"), (payload, scale))
+    out = torch.empty(payload.shape, dtype=torch.float32, device=payload.device)
+    if base == "vblock" and checkpoint.tile_size == VBLOCK and payload.dtype != torch.int8:
+        host.call(_ENTRY["gdnr_dequantize_vblock32"], (payload, scale, out), (), (), None)
+    else:
+        host.call(_ENTRY["gdnr_dequantize_checkpoint"], (payload, scale, out), (code, checkpoint.tile_size), (), None)
     return out
 
 
@@ -166,9 +160,21 @@ def dequantize_checkpoint(checkpoint: QuantizedCheckpoint) -> torch.Tensor:
 # Operators
 # ---------------------------------------------------------------------------
 
-def _new_out(q: torch.Tensor, v_cache: torch.Tensor) -> torch.Tensor:
+# argument names of the operators' tensors, as their device check reports them
+_REPLAY_NAMES = ("checkpoint", "checkpoint_scale", "q", "k_cache", "v_cache", "g_cache", "beta_cache", "valid_len",
+                 "flush", "out")
+_SPLIT_NAMES = ("checkpoint", "checkpoint_scale", "q", "k_cache", "v_cache", "g_cache", "beta_cache", "valid_len",
+                "transformed_query_buffer", "coefficient_buffer", "out")
+_PREP_NAMES = ("mixed_qkv", "a", "b", "a_log", "dt_bias", "pos", "q_out", "k_ring", "v_ring", "g_ring", "beta_ring")
+_STEP_NAMES = ("mixed_qkv", "a", "b", "a_log", "dt_bias", "pos", "checkpoint", "checkpoint_scale", "q_out", "k_ring",
+               "v_ring", "g_ring", "beta_ring", "valid_len", "flush", "out", "state_indices")
+_RMW_NAMES = ("state", "q", "k", "v", "g", "beta")
+_RMW_PACKED_NAMES = ("mixed_qkv", "a", "b", "a_log", "dt_bias", "initial_state", "ssm_state_indices", "out")
+
+
+def _new_out(host, q: torch.Tensor, v_cache: torch.Tensor) -> torch.Tensor:
     batch, _, value_heads, value_dim = v_cache.shape
-    return torch.empty(batch, value_heads, value_dim, dtype=q.dtype, device=q.device)
+    return host.empty(q, (batch, value_heads, value_dim))
 
 
 def gdn_replay_fp8(
@@ -192,15 +198,12 @@ def gdn_replay_fp8(
     (reference quantiser semantics, ref:36-37,83-99). Returns out [B,HV,V]
     (allocated with q's dtype when not given)."""
     del num_warps
-    device = _require_cuda(checkpoint=checkpoint, checkpoint_scale=checkpoint_scale, q=q, k_cache=k_cache,
-                           v_cache=v_cache, g_cache=g_cache, beta_cache=beta_cache, valid_len=valid_len,
-                           flush=flush, out=out)
-    output = _new_out(q, v_cache) if out is None else out
-    with torch.cuda.device(device):
-        gdnr_lib.call("gdnr_replay_fp8",
-                      [checkpoint, checkpoint_scale, q, k_cache, v_cache, g_cache, beta_cache,
-                       _as_i32(valid_len), _as_flag(flush), output],
-                      [block_v], gdnr_lib.current_stream(device))
+    host = gdnr_lib.host()
+    host.require(_REPLAY_NAMES, (checkpoint, checkpoint_scale, q, k_cache, v_cache, g_cache, beta_cache, valid_len,
+                                 flush, out))
+    output = _new_out(host, q, v_cache) if out is None else out
+    host.call(_REPLAY, (checkpoint, checkpoint_scale, q, k_cache, v_cache, g_cache, beta_cache, _as_i32(valid_len),
+                        _as_flag(flush), output), (block_v,), (), None)
     return output
 
 
@@ -227,16 +230,13 @@ def gdn_replay_fp8_split(
     coefficient_buffer [B,HV,>=L] f32 (t < valid_len only), then streams the
     checkpoint. Same output as gdn_replay_fp8 with flush = 0."""
     del num_warps, num_stages
-    device = _require_cuda(checkpoint=checkpoint, checkpoint_scale=checkpoint_scale, q=q, k_cache=k_cache,
-                           v_cache=v_cache, g_cache=g_cache, beta_cache=beta_cache, valid_len=valid_len,
-                           transformed_query_buffer=transformed_query_buffer,
-                           coefficient_buffer=coefficient_buffer, out=out)
-    output = _new_out(q, v_cache) if out is None else out
-    with torch.cuda.device(device):
-        gdnr_lib.call("gdnr_replay_fp8_split",
-                      [checkpoint, checkpoint_scale, q, k_cache, v_cache, g_cache, beta_cache,
-                       _as_i32(valid_len), transformed_query_buffer, coefficient_buffer, output],
-                      [block_v, block_kc, int(bool(precompute_grouped))], gdnr_lib.current_stream(device))
+    host = gdnr_lib.host()
+    host.require(_SPLIT_NAMES, (checkpoint, checkpoint_scale, q, k_cache, v_cache, g_cache, beta_cache, valid_len,
+                                transformed_query_buffer, coefficient_buffer, out))
+    output = _new_out(host, q, v_cache) if out is None else out
+    host.call(_SPLIT, (checkpoint, checkpoint_scale, q, k_cache, v_cache, g_cache, beta_cache, _as_i32(valid_len),
+                       transformed_query_buffer, coefficient_buffer, output),
+              (block_v, block_kc, int(bool(precompute_grouped))), (), None)
     return output
 
 
@@ -260,13 +260,10 @@ def gdn_prep_ring(
     dt_bias), beta = sigmoid(b) -> ring slot pos[b]. A_log and dt_bias are
     read as float32 (converted when given otherwise)."""
     del num_warps
-    device = _require_cuda(mixed_qkv=mixed_qkv, a=a, b=b, a_log=a_log, dt_bias=dt_bias, pos=pos, q_out=q_out,
-                           k_ring=k_ring, v_ring=v_ring, g_ring=g_ring, beta_ring=beta_ring)
-    with torch.cuda.device(device):
-        gdnr_lib.call("gdnr_prep_ring",
-                      [mixed_qkv, a, b, a_log.float(), dt_bias.float(), _as_i32(pos), q_out, k_ring, v_ring,
-                       g_ring, beta_ring],
-                      [int(bool(fused))], gdnr_lib.current_stream(device))
+    host = gdnr_lib.host()
+    host.require(_PREP_NAMES, (mixed_qkv, a, b, a_log, dt_bias, pos, q_out, k_ring, v_ring, g_ring, beta_ring))
+    host.call(_PREP, (mixed_qkv, a, b, _as_f32(a_log), _as_f32(dt_bias), _as_i32(pos), q_out, k_ring, v_ring, g_ring,
+                      beta_ring), (int(bool(fused)),), (), None)
 
 
 def gdn_prep_replay_fp8(
@@ -299,26 +296,18 @@ def gdn_prep_replay_fp8(
     rings are a slot-indexed cache [S, ...] (vLLM's layout, slot 0 the null
     slot) and batch entry b uses slot state_indices[b]; the other arguments
     stay per batch entry (gdnr_prep_replay_fp8_slots)."""
-    device = _require_cuda(mixed_qkv=mixed_qkv, a=a, b=b, a_log=a_log, dt_bias=dt_bias, pos=pos,
-                           checkpoint=checkpoint, checkpoint_scale=checkpoint_scale, q_out=q_out, k_ring=k_ring,
-                           v_ring=v_ring, g_ring=g_ring, beta_ring=beta_ring, valid_len=valid_len, flush=flush,
-                           out=out, state_indices=state_indices)
-    batch = mixed_qkv.shape[0]
-    output = (torch.empty(batch, v_ring.shape[2], v_ring.shape[3], dtype=q_out.dtype, device=device)
-              if out is None else out)
-    with torch.cuda.device(device):
-        if state_indices is None:
-            gdnr_lib.call("gdnr_prep_replay_fp8",
-                          [mixed_qkv, a, b, a_log.float(), dt_bias.float(), _as_i32(pos), checkpoint,
-                           checkpoint_scale, q_out, k_ring, v_ring, g_ring, beta_ring, _as_i32(valid_len),
-                           _as_flag(flush), output],
-                          [block_v], gdnr_lib.current_stream(device))
-        else:
-            gdnr_lib.call("gdnr_prep_replay_fp8_slots",
-                          [mixed_qkv, a, b, a_log.float(), dt_bias.float(), _as_i32(pos), _as_i32(state_indices),
-                           checkpoint, checkpoint_scale, q_out, k_ring, v_ring, g_ring, beta_ring,
-                           _as_i32(valid_len), _as_flag(flush), output],
-                          [block_v], gdnr_lib.current_stream(device))
+    host = gdnr_lib.host()
+    host.require(_STEP_NAMES, (mixed_qkv, a, b, a_log, dt_bias, pos, checkpoint, checkpoint_scale, q_out, k_ring,
+                               v_ring, g_ring, beta_ring, valid_len, flush, out, state_indices))
+    output = (host.empty(q_out, (mixed_qkv.shape[0], v_ring.shape[2], v_ring.shape[3])) if out is None else out)
+    if state_indices is None:
+        host.call(_STEP, (mixed_qkv, a, b, _as_f32(a_log), _as_f32(dt_bias), _as_i32(pos), checkpoint,
+                          checkpoint_scale, q_out, k_ring, v_ring, g_ring, beta_ring, _as_i32(valid_len),
+                          _as_flag(flush), output), (block_v,), (), None)
+    else:
+        host.call(_STEP_SLOTS, (mixed_qkv, a, b, _as_f32(a_log), _as_f32(dt_bias), _as_i32(pos),
+                                _as_i32(state_indices), checkpoint, checkpoint_scale, q_out, k_ring, v_ring, g_ring,
+                                beta_ring, _as_i32(valid_len), _as_flag(flush), output), (block_v,), (), None)
     return output
 
 
@@ -336,10 +325,10 @@ def gdn_bf16_step(
     q's dtype. state [B,HV,V,K] (bf16, f16 or f32); q, k [B,H,K];
     v [B,HV,V]; g, beta [B,HV] -- views with unit inner stride are taken as
     they are (the reference passes ring slices, bench_gdn_replayssm.py:278-287)."""
-    device = _require_cuda(state=state, q=q, k=k, v=v, g=g, beta=beta)
-    output = torch.empty(state.shape[0], state.shape[1], state.shape[2], dtype=q.dtype, device=device)
-    with torch.cuda.device(device):
-        gdnr_lib.call("gdnr_bf16_step", [state, q, k, v, g, beta, output], [], gdnr_lib.current_stream(device))
+    host = gdnr_lib.host()
+    host.require(_RMW_NAMES, (state, q, k, v, g, beta))
+    output = host.empty(q, tuple(state.shape[:3]))
+    host.call(_RMW, (state, q, k, v, g, beta, output), (), (), None)
     return output
 
 
@@ -359,16 +348,11 @@ def gdn_bf16_step_packed(
     initial_state [slots, HV, V, K] updated in place at slot
     ssm_state_indices[b] (slot 0 the null slot), out [B, 1, HV, V] =
     scale (S q); scale defaults to head_k_dim ** -0.5, as vLLM passes it."""
-    device = _require_cuda(mixed_qkv=mixed_qkv, a=a, b=b, a_log=a_log, dt_bias=dt_bias,
-                           initial_state=initial_state, ssm_state_indices=ssm_state_indices, out=out)
-    batch = mixed_qkv.shape[0]
+    host = gdnr_lib.host()
+    host.require(_RMW_PACKED_NAMES, (mixed_qkv, a, b, a_log, dt_bias, initial_state, ssm_state_indices, out))
     if out is None:
-        out = torch.empty(batch, 1, initial_state.shape[1], initial_state.shape[2], dtype=mixed_qkv.dtype,
-                          device=device)
-    with torch.cuda.device(device):
-        gdnr_lib.call("gdnr_bf16_step_packed", [mixed_qkv, a, b, a_log.float(), dt_bias.float(), initial_state,
-                                                _as_i32(ssm_state_indices), out], [],
-                      gdnr_lib.current_stream(device),
-                      floats=[initial_state.shape[-1] ** -0.5 if scale is None else scale])
+        out = host.empty(mixed_qkv, (mixed_qkv.shape[0], 1, initial_state.shape[1], initial_state.shape[2]))
+    host.call(_RMW_PACKED, (mixed_qkv, a, b, _as_f32(a_log), _as_f32(dt_bias), initial_state,
+                            _as_i32(ssm_state_indices), out), (),
+              (initial_state.shape[-1] ** -0.5 if scale is None else scale,), None)
     return out
-

@@ -6,7 +6,8 @@ Objects go to _build/ next to this file; the library is written in-tree
 (next to this file) so it travels with the source tree to the GPU host.
 The C-ABI validation layer (csrc/gdnr_abi.cpp) is plain C++ compiled by g++;
 the kernels (csrc/*.hip) by hipcc. Packed-FP32 VALU instructions
-are disabled for all device code.
+are disabled for all device code. The host extension module _gdnr_host.so
+(csrc/gdnr_host.cpp, g++ with torch's headers) is written next to the library.
 """
 
 from __future__ import annotations
@@ -15,6 +16,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -23,9 +25,11 @@ CSRC = PKG_DIR / "csrc"
 INCLUDE = PKG_DIR.parent / "include"
 BUILD_DIR = PKG_DIR / "_build"
 LIBRARY = PKG_DIR / "libgdnreplay.so"
+HOST_MODULE = PKG_DIR / "_gdnr_host.so"
 ARCH = os.environ.get("GDNR_OFFLOAD_ARCH", "gfx950")
 
-HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+ROCM = Path("/opt/rocm")
+HIPCC = shutil.which("hipcc") or str(ROCM / "bin/hipcc")
 DEVICE_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -57,6 +61,18 @@ def _run(cmd: list[str], verbose: bool) -> None:
         print(stderr, file=sys.stderr)
 
 
+def _host_module_job(out: Path) -> list[str]:
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    return ["g++", *HOST_FLAGS, "-Wno-unused-parameter", "-shared", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{INCLUDE}",
+            f"-I{sysconfig.get_paths()['include']}", f"-isystem{root / 'include'}",
+            f"-isystem{root / 'include/torch/csrc/api/include'}", f"-isystem{ROCM / 'include'}",
+            str(CSRC / "gdnr_host.cpp"), "-o", str(out), f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10",
+            "-lc10_hip"]
+
+
 def build(verbose: bool = False) -> Path:
     BUILD_DIR.mkdir(exist_ok=True)
     inc = [f"-I{INCLUDE}", f"-I{CSRC}"]
@@ -73,6 +89,8 @@ def build(verbose: bool = False) -> Path:
         jobs.append([HIPCC, *DEVICE_FLAGS, *inc, "-c", str(CSRC / f"{src}.hip"), "-o", str(obj)])
     abi_obj = BUILD_DIR / "gdnr_abi.o"
     jobs.append(["g++", *HOST_FLAGS, *inc, "-c", str(CSRC / "gdnr_abi.cpp"), "-o", str(abi_obj)])
+    host_tmp = HOST_MODULE.with_name(HOST_MODULE.name + ".tmp")
+    jobs.append(_host_module_job(host_tmp))
     with ThreadPoolExecutor(max_workers=len(jobs)) as pool:
         for future in [pool.submit(_run, cmd, verbose) for cmd in jobs]:
             future.result()
@@ -80,6 +98,7 @@ def build(verbose: bool = False) -> Path:
     _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, kern_objs), str(abi_obj), "-o", str(tmp)],
          verbose)
     tmp.replace(LIBRARY)
+    host_tmp.replace(HOST_MODULE)
     return LIBRARY
 
 

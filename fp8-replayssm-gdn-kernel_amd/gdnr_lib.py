@@ -1,16 +1,19 @@
-"""ctypes bindings of libgdnreplay.so (the C ABI declared in include/gdnr.h).
+"""Bindings of libgdnreplay.so (the C ABI declared in include/gdnr.h).
 
 Tensors cross the boundary as ``gdnr_tensor`` descriptors (device pointer,
-dtype code, shape, element strides). Every call enqueues on the caller's
-current HIP stream and returns without synchronising; a nonzero status is
-raised as ``GdnrError`` with the library's own message.
+dtype code, shape, element strides), which the extension module _gdnr_host
+(csrc/gdnr_host.cpp) fills; the library itself is loaded by ctypes and its
+entry points' addresses bound to the extension. Every call enqueues on the
+caller's current HIP stream and returns without synchronising; a nonzero
+status is raised as ``GdnrError`` with the library's own message.
 
-There is no fallback: if the library is not built, the first call raises.
+There is no fallback: if either is not built, the first call raises.
 """
 
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 from pathlib import Path
 
@@ -18,6 +21,7 @@ import torch
 
 PKG_DIR = Path(__file__).resolve().parent
 LIBRARY_PATH = Path(os.environ.get("GDNR_LIBRARY", PKG_DIR / "libgdnreplay.so"))
+HOST_PATH = PKG_DIR / "_gdnr_host.so"
 
 MAX_DIMS = 4
 ABI_VERSION = 1
@@ -73,7 +77,11 @@ ENTRY_POINTS = {
     "gdnr_stream_probe": (1, 1),
 }
 
+# position of each entry point in the extension's table
+ENTRY_IDS = {name: i for i, name in enumerate(ENTRY_POINTS)}
+
 _lib = None
+_host = None
 
 
 def load_library(path: Path | None = None) -> ctypes.CDLL:
@@ -108,34 +116,33 @@ def load_library(path: Path | None = None) -> ctypes.CDLL:
     return lib
 
 
-def describe(t: torch.Tensor | None) -> GdnrTensor | None:
-    """gdnr_tensor descriptor of a torch tensor (None stays None)."""
-    if t is None:
-        return None
-    if t.dim() > MAX_DIMS:
-        raise ValueError(f"tensors of rank {t.dim()} are not accepted")
-    code = DTYPE_CODES.get(t.dtype)
-    if code is None:
-        raise TypeError(f"dtype {t.dtype} is not accepted by libgdnreplay")
-    desc = GdnrTensor()
-    desc.data = t.data_ptr() if t.numel() else None
-    desc.dtype = code
-    desc.ndim = t.dim()
-    for d in range(t.dim()):
-        desc.shape[d] = t.shape[d]
-        desc.strides[d] = t.stride(d)
-    return desc
+def host():
+    """The extension module _gdnr_host with the library's entry points bound
+    (loaded once). Raises if it or the library is not built."""
+    global _host
+    if _host is None:
+        lib = load_library()
+        if not HOST_PATH.exists():
+            raise RuntimeError(
+                f"{HOST_PATH} is not built; run `python {PKG_DIR / 'gdnr_build.py'}` (the HIP path has no fallback)")
+        spec = importlib.util.spec_from_file_location("_gdnr_host", HOST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+
+        def address(name: str) -> int:
+            return ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
+
+        module.bind(GdnrError, address("gdnr_last_error"),
+                    [(address(name), n_tensors, n_ints, sum(n_floats))
+                     for name, (n_tensors, n_ints, *n_floats) in ENTRY_POINTS.items()])
+        _host = module
+    return _host
 
 
 def call(name: str, tensors, ints=(), stream: int | None = None, floats=()) -> None:
-    """Invoke an entry point; tensors must already be on the same CUDA device."""
-    lib = load_library()
-    fn = getattr(lib, name)
-    descs = [describe(t) for t in tensors]
-    ptrs = [ctypes.byref(d) if d is not None else None for d in descs]
-    status = fn(*ptrs, *[int(i) for i in ints], *[float(x) for x in floats], ctypes.c_void_p(stream))
-    if status != 0:
-        raise GdnrError(status, lib.gdnr_last_error().decode())
+    """Invoke an entry point; tensors must already be on the same CUDA device.
+    stream: a hipStream_t (None: torch's current stream on that device)."""
+    host().call(ENTRY_IDS[name], tuple(tensors), tuple(int(i) for i in ints), tuple(float(x) for x in floats), stream)
 
 
 def current_stream(device: torch.device) -> int:
