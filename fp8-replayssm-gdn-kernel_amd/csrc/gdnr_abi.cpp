@@ -691,25 +691,16 @@ int check_quant(const gdnr_tensor* state, const gdnr_tensor* payload, const gdnr
   return check_shape(scale, "scale", {*B, *HV, *V / gdnr::kVBlock});
 }
 
-void fill_quant(gdnr::QuantArgs* q, const gdnr_tensor* state, const gdnr_tensor* payload, const gdnr_tensor* scale,
-                int64_t B, int64_t HV, int64_t V) {
-  q->state = (const float*)state->data;
-  q->st_b = state->strides[0];
-  q->st_h = state->strides[1];
-  q->st_v = state->strides[2];
-  q->codes = (uint8_t*)payload->data;
-  q->ck_b = payload->strides[0];
-  q->ck_h = payload->strides[1];
-  q->ck_v = payload->strides[2];
-  q->scale = scale->data;
-  q->sc_b = scale->strides[0];
-  q->sc_h = scale->strides[1];
-  q->sc_v = scale->strides[2];
-  q->scale_dt = scale->dtype;
-  q->saturated = nullptr;
-  q->B = (int32_t)B;
-  q->HV = (int32_t)HV;
-  q->V = (int32_t)V;
+// the vblock32 format of validated tensors (check_quant)
+gdnr::FormatArgs vblock32_format(const gdnr_tensor* state, const gdnr_tensor* payload, const gdnr_tensor* scale) {
+  gdnr::FormatArgs f = {};
+  f.state = (float*)state->data, f.st_b = state->strides[0], f.st_h = state->strides[1], f.st_v = state->strides[2];
+  f.payload = payload->data, f.pl_b = payload->strides[0], f.pl_h = payload->strides[1], f.pl_v = payload->strides[2];
+  f.scale = scale->data, f.sc_b = scale->strides[0], f.sc_h = scale->strides[1], f.sc_r = scale->strides[2];
+  f.scale_dt = scale->dtype == GDNR_DTYPE_F32 ? gdnr::DT_F32 : gdnr::DT_F16;
+  f.B = (int32_t)state->shape[0], f.HV = (int32_t)state->shape[1], f.V = (int32_t)state->shape[2];
+  f.K = gdnr::kKeyDim, f.gran = gdnr::kGranVblock, f.tile = gdnr::kVBlock;
+  return f;
 }
 
 }  // namespace
@@ -1077,15 +1068,12 @@ int gdnr_quantize_vblock32(const gdnr_tensor* state, const gdnr_tensor* payload,
     GDNR_TRY(check_shape(saturated, "saturated", {B, HV, V / gdnr::kVBlock}));
   }
   if (B * HV * V == 0) return GDNR_OK;
-  gdnr::QuantArgs q = {};
-  fill_quant(&q, state, payload, scale, B, HV, V);
+  gdnr::FormatArgs f = vblock32_format(state, payload, scale);
   if (saturated) {
-    q.saturated = (int32_t*)saturated->data;
-    q.sa_b = saturated->strides[0];
-    q.sa_h = saturated->strides[1];
-    q.sa_v = saturated->strides[2];
+    f.saturated = (int32_t*)saturated->data;
+    f.sa_b = saturated->strides[0], f.sa_h = saturated->strides[1], f.sa_r = saturated->strides[2];
   }
-  return hip_status(gdnr::launch_quantize(q, stream));
+  return hip_status(gdnr::launch_format_quantize(f, stream));
 }
 
 int gdnr_dequantize_vblock32(const gdnr_tensor* payload, const gdnr_tensor* scale, const gdnr_tensor* state,
@@ -1094,9 +1082,7 @@ int gdnr_dequantize_vblock32(const gdnr_tensor* payload, const gdnr_tensor* scal
   int64_t B, HV, V;
   GDNR_TRY(check_quant(state, payload, scale, &B, &HV, &V));
   if (B * HV * V == 0) return GDNR_OK;
-  gdnr::QuantArgs q = {};
-  fill_quant(&q, state, payload, scale, B, HV, V);
-  return hip_status(gdnr::launch_dequantize(q, stream));
+  return hip_status(gdnr::launch_format_dequantize(vblock32_format(state, payload, scale), stream));
 }
 
 int gdnr_stream_probe(const gdnr_tensor* buffer, int32_t flags, void* stream) {

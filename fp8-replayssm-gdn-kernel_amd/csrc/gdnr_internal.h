@@ -115,14 +115,6 @@ struct PrepArgs {
   int32_t B, H, HV, G, V, L;
 };
 
-struct QuantArgs {
-  const float* state; int64_t st_b, st_h, st_v;   // quantise reads, dequantise writes (as float*)
-  uint8_t* codes; int64_t ck_b, ck_h, ck_v;
-  void* scale; int64_t sc_b, sc_h, sc_v; int32_t scale_dt;
-  int32_t* saturated; int64_t sa_b, sa_h, sa_v;   // may be null
-  int32_t B, HV, V;
-};
-
 // Checkpoint formats of the reference quantiser (gdnr_formats.hip): scale
 // group granularity, tile size (tile / vblock), fp8 or int8 codes. Strides
 // in elements; the scale and saturated tensors are indexed [b, hv, i, j]
@@ -198,12 +190,10 @@ int device_cus();
 // symbol cannot be resolved).
 constexpr int64_t kSplitScratchBytes = 3 << 20;
 uint8_t* split_scratch();
-int launch_quantize(const QuantArgs& a, void* stream);
 int launch_rmw_step(const RmwArgs& a, int state_dt, int act_dt, void* stream);
 int launch_rmw_packed(const RmwArgs& a, int state_dt, int act_dt, bool gate_f32, void* stream);
 int launch_format_quantize(const FormatArgs& a, void* stream);
 int launch_format_dequantize(const FormatArgs& a, void* stream);
-int launch_dequantize(const QuantArgs& a, void* stream);
 // coalesced stream over bytes (a multiple of 16) at buf: read only, or read
 // and written back in place; plain or non-temporal loads; chunked: read only,
 // in the decode kernel's order (a 16 KiB chunk per wave, 16 loads in flight),

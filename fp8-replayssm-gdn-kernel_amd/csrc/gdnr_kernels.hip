@@ -13,16 +13,15 @@
 //   5. the checkpoint matvec o = (codes . T) * scale on the VALU (no MFMA:
 //      one FMA per byte), rows reduced across 8 lanes with DPP.
 // The order of steps 2-3 is pinned with compiler fences.
-// These kernels serve the split path, the standalone prep, the quantiser and
-// the rings that the others leave: longer than 16 tokens with f32
+// These kernels serve the split path, the standalone prep and the rings that the others leave: longer than 16 tokens with f32
 // activations (or a V the ring kernel does not hold, or tensors past its
 // 32-bit offsets). Rings of up to 16 tokens go through the decode kernel
 // (gdnr_decode.hip, 16-bit activations) or the step kernel (gdnr_step.hip,
 // f32 activations), longer ones of 16-bit activations through the decode
 // kernel (small batches) or the ring kernel (gdnr_ring.hip).
 //
-// This file is compiled once per activation dtype: GDNR_ACT=0 (bf16, also
-// holds the dtype-free quantiser kernels), 1 (f16), 2 (f32).
+// This file is compiled once per activation dtype: GDNR_ACT=0 (bf16), 1
+// (f16), 2 (f32).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -581,109 +580,6 @@ __global__ __launch_bounds__(256) void prep_kernel(const PrepArgs a) {
   }
 }
 
-#if GDNR_ACT == 0
-// vblock32 quantiser (reference ref:36-37,71-99): one wave per 32 x 128 block.
-__global__ __launch_bounds__(256) void quantize_kernel(const QuantArgs a) {
-  const int lane = threadIdx.x & 63;
-  const int nvb = a.V / kVBlock;
-  const int item = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
-  if (item >= a.B * a.HV * nvb) return;
-  const int vb = item % nvb;
-  const int hv = (item / nvb) % a.HV;
-  const int b = item / (nvb * a.HV);
-  const int gi = lane & 7, gm = lane >> 3;
-  const float* src = a.state + (int64_t)b * a.st_b + (int64_t)hv * a.st_h + (int64_t)(vb * kVBlock + gm) * a.st_v + 16 * gi;
-  float x[4][16];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const float4* p = (const float4*)(src + (int64_t)(8 * j) * a.st_v);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float4 w = p[i];
-      x[j][4 * i] = w.x;
-      x[j][4 * i + 1] = w.y;
-      x[j][4 * i + 2] = w.z;
-      x[j][4 * i + 3] = w.w;
-    }
-  }
-  uint32_t am = 0;
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) am = max(am, __float_as_uint(x[j][e]) & 0x7FFFFFFFu);
-  am = wave_max_u32(am);
-  const float amax = __uint_as_float(am);
-  const float s32 = (amax > 0.0f) ? amax / 448.0f : 1.0f;
-  int sat = 0;
-  uint8_t* dst = a.codes + (int64_t)b * a.ck_b + (int64_t)hv * a.ck_h + (int64_t)(vb * kVBlock + gm) * a.ck_v + 16 * gi;
-  // quotients x / s32 as IEEE division rounds them: quotient_rn when the
-  // block is finite (|x / s32| <= 448 (1 + 2^-23): no clamp needed), else
-  // the division with the reference's clamp and NaN encoding
-  const bool fast = quotient_fast(am, s32);
-  const float r = 1.0f / s32;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    float y[16];
-    uint4 w;
-    if (fast) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        y[e] = quotient_rn(x[j][e], s32, r);
-        sat += fabsf(y[e]) > 448.0f ? 1 : 0;
-      }
-      w.x = f32x4_to_fp8(y[0], y[1], y[2], y[3]);
-      w.y = f32x4_to_fp8(y[4], y[5], y[6], y[7]);
-      w.z = f32x4_to_fp8(y[8], y[9], y[10], y[11]);
-      w.w = f32x4_to_fp8(y[12], y[13], y[14], y[15]);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        y[e] = x[j][e] / s32;
-        sat += fabsf(y[e]) > 448.0f ? 1 : 0;
-      }
-      w.x = f32x4_to_fp8_ref(y[0], y[1], y[2], y[3]);
-      w.y = f32x4_to_fp8_ref(y[4], y[5], y[6], y[7]);
-      w.z = f32x4_to_fp8_ref(y[8], y[9], y[10], y[11]);
-      w.w = f32x4_to_fp8_ref(y[12], y[13], y[14], y[15]);
-    }
-    *(uint4*)(dst + (int64_t)(8 * j) * a.ck_v) = w;
-  }
-  sat = wave_sum_i32(sat);
-  if (lane == 0) {
-    st_dt(a.scale, (int64_t)b * a.sc_b + (int64_t)hv * a.sc_h + (int64_t)vb * a.sc_v, a.scale_dt, (float)(_Float16)s32);
-    if (a.saturated) a.saturated[(int64_t)b * a.sa_b + (int64_t)hv * a.sa_h + (int64_t)vb * a.sa_v] = sat;
-  }
-}
-
-// state = float(code) * float(scale) (reference ref:109-134).
-__global__ __launch_bounds__(256) void dequantize_kernel(const QuantArgs a) {
-  const int lane = threadIdx.x & 63;
-  const int nvb = a.V / kVBlock;
-  const int item = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
-  if (item >= a.B * a.HV * nvb) return;
-  const int vb = item % nvb;
-  const int hv = (item / nvb) % a.HV;
-  const int b = item / (nvb * a.HV);
-  const int gi = lane & 7, gm = lane >> 3;
-  const float sc = ld_dt(a.scale, (int64_t)b * a.sc_b + (int64_t)hv * a.sc_h + (int64_t)vb * a.sc_v, a.scale_dt);
-  const uint8_t* src = a.codes + (int64_t)b * a.ck_b + (int64_t)hv * a.ck_h + (int64_t)(vb * kVBlock + gm) * a.ck_v + 16 * gi;
-  float* dst = (float*)a.state + (int64_t)b * a.st_b + (int64_t)hv * a.st_h + (int64_t)(vb * kVBlock + gm) * a.st_v + 16 * gi;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const uint4 w = *(const uint4*)(src + (int64_t)(8 * j) * a.ck_v);
-    const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
-    float4* d = (float4*)(dst + (int64_t)(8 * j) * a.st_v);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float f[4];
-      fp8x4_to_f32(ws[i], f);
-      d[i] = make_float4(f[0] * sc, f[1] * sc, f[2] * sc, f[3] * sc);
-    }
-  }
-}
-
-#endif  // GDNR_ACT == 0
-
 // ------------------------------------------------------------------ launch
 int finish_launch() {
   const hipError_t e = hipGetLastError();
@@ -741,18 +637,6 @@ int GDNR_SUFFIX(launch_prep)(const PrepArgs& a, bool gate_f32, void* stream) {
 }
 
 #if GDNR_ACT == 0
-int launch_quantize(const QuantArgs& a, void* stream) {
-  const int items = a.B * a.HV * (a.V / kVBlock);
-  hipLaunchKernelGGL(quantize_kernel, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, (hipStream_t)stream, a);
-  return finish_launch();
-}
-
-int launch_dequantize(const QuantArgs& a, void* stream) {
-  const int items = a.B * a.HV * (a.V / kVBlock);
-  hipLaunchKernelGGL(dequantize_kernel, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, (hipStream_t)stream, a);
-  return finish_launch();
-}
-
 const char* hip_error_string(int code) { return hipGetErrorString((hipError_t)code); }
 #endif
 
