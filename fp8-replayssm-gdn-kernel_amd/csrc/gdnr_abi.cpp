@@ -574,12 +574,15 @@ int launch_ring(const gdnr::ReplayArgs& r, int act, bool fused, bool gate_f32, v
   // unit on (what is resident at once); four of 32 rows below that, where
   // twice the workgroups fill the chip and a flush is half as long. us per
   // step with staggered fills, four and two waves: B=24, L=64 11.9 and 14.6;
-  // B=37, L=48 14.7 and 18.6; B=64, L=64 22.0 and 21.7; B=256 73 and 54.
+  // B=37, L=48 14.7 and 18.6; B=64, L=64 22.0 and 21.7; B=256 73 and 54
+  // (with the flushes whole).
   const int64_t resident = 3 * (int64_t)gdnr::device_cus();
   a.nwh = a.V == 256 || a.G % 2 || (a.V == 128 && (int64_t)a.B * a.H * (a.G / 2) <= resident) ? 4 : 2;
   a.gw = 4 / a.nwh;
   a.units = a.G / a.gw;  // head groups per key head
   // flushing sequences first, where the workgroups take more than one round
+  // (in one round it only costs the replays: B=24, L=64 at fill 32 9.4 against
+  // 8.9)
   a.seq_major = a.flush && a.B <= gdnr::kRingOrder && (int64_t)a.B * a.H * a.units > resident;
   if (act == GDNR_DTYPE_BF16) return gdnr::launch_ring_bf16(a, fused, gate_f32, stream);
   return gdnr::launch_ring_f16(a, fused, gate_f32, stream);

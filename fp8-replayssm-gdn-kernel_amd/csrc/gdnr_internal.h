@@ -72,6 +72,7 @@ constexpr int32_t kMaxStepLds = 160 * 1024;  // gfx950 LDS per workgroup
 constexpr int kStepRing = 16;                // ring capacity handled by the step kernel
 constexpr int kDecodeChunks = 4;             // chunks of kStepRing tokens of the decode kernel's longest ring
 constexpr int kRingOrder = 256;               // sequences the ring kernel orders (flushes first)
+constexpr int kRingHalves = 8;                // flushing sequences it gives two workgroups each
 constexpr uint32_t kWaitPolls = 1u << 22;     // default poll budget of a bounded LDS wait
 
 // Argument block of the step kernel (gdnr_step.hip), built on the host from a

@@ -12,11 +12,11 @@
 // coefficient chain) overlaps the others' streams.
 //
 // Bound: a replay at full batch by its bytes and its VALU issue (B=64, L=64,
-// fill 32: 60 MB in 17.1 us, 3.5 TB/s, against 25.3 for the per-token chain of
-// gdnr_kernels.hip that this kernel replaces; fill 63 21.6 against 36.0); a
+// fill 32: 60 MB in 17.4 us, 3.5 TB/s, against 25.3 for the per-token chain of
+// gdnr_kernels.hip that this kernel replaces; fill 63 22.1 against 36.0); a
 // flush by its waves' own latency (6 us to the factors, then 3.7 us a tile: a
 // launch of 24 flushes 25 us against 192). A step of B=64, L=64 with one
-// sequence flushing takes 21.7 us against 140.
+// sequence flushing takes 18.0 us against 140.
 //
 // Replay (the adjoint of the reference's reverse chain,
 // prototype/gdn_replayssm_fp8_kernel.py:121-173, in Gram form over the whole
@@ -43,6 +43,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #ifndef GDNR_ACT
@@ -128,7 +129,9 @@ __device__ __forceinline__ void lds_barrier() {
 __device__ __forceinline__ constexpr int gram_tile(int r, int c) { return kLdsG + (c * (c + 1) / 2 + r) * 16 * kGS * 4; }
 
 template <int VB, int WPH, bool FUSED, bool GATE_F32, bool SLOTS>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) void ring_kernel(const StepArgs a) {
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) void ring_kernel(
+    const uint8_t* m_len, const uint8_t* m_pos, const uint8_t* m_flush, uint32_t m_vs, uint32_t m_ps, uint32_t m_fs,
+    int32_t m_L, int32_t m_grp, int32_t m_order, int32_t m_G, const StepArgs a) {
   constexpr int ES = 2;
   constexpr int GW = NW / WPH;            // value heads per workgroup
   constexpr int RPW = 32 * VB;            // V-rows per wave
@@ -137,24 +140,27 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
   const int lane = threadIdx.x & 63;
   const int q4 = lane >> 4, l16 = lane & 15;
   const int w = uni(threadIdx.x >> 6);
-  const int n_grp = a.units;              // head groups per key head
+  const int n_grp = m_grp;              // head groups per key head
   const int r = blockIdx.x;
   const int h = uni(r / n_grp), grp = r - h * n_grp;
   const int j = w / WPH, part = w % WPH;  // value head in the workgroup, row block of it
-  const int hv = h * a.G + grp * GW + j;
+  const int hv = h * m_G + grp * GW + j;
   const int R0 = RPW * part;
 
   // ---- the sequence and its metadata: how much of the ring to read is known
-  // before any of it is requested. A launch that may hold flushes takes the
-  // flushing sequences first (a flush runs longer than a replay, and one that
-  // starts in the last round of workgroups ends the launch late: B=64, L=64
-  // with one flush a step 21.7 us against 27.8): the blockIdx.y-th sequence
-  // of that order, found from every sequence's flag, whose lane holds its
-  // metadata too. Larger batches (a few flushes a launch at least, in rounds
-  // enough) keep their order.
+  // before any of it is requested. (These arguments are preloaded into SGPRs
+  // at wave launch.) A launch that may hold flushes and takes more than one
+  // round of workgroups (m_order: 1 + the grid's rows past the batch) takes
+  // the flushing sequences first, and a few of them with two workgroups each:
+  // a flush runs longer than a replay, and one that starts in the last round
+  // ends the launch late. B=64, L=64, one flush a step: 27.8 us in the batch's
+  // order, 21.1 flushes first, 18.0 in halves too (replays alone 17.4). The
+  // blockIdx.y-th sequence of that order is found from every sequence's flag;
+  // its lane holds its metadata too.
   int b = blockIdx.y, bs = b, n, pos = -1;
-  bool do_flush = false;
-  if (a.seq_major) {
+  bool do_flush = false, split = false, spare = false;
+  int half = 0;
+  if (m_order) {
     constexpr int NO = kRingOrder / 64;
     uint32_t f[NO];
     int vl[NO], ps[NO], sl[NO];
@@ -162,9 +168,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
     for (int i = 0; i < NO; ++i) {
       if (64 * i >= a.B) break;
       const uint32_t bq = (uint32_t)min(64 * i + lane, a.B - 1);
-      f[i] = a.flush[bq * a.fl_s];
-      vl[i] = *(const int*)(a.valid_len + bq * a.vl_s);
-      if constexpr (FUSED) ps[i] = *(const int*)(a.pos + bq * a.pos_s);
+      f[i] = m_flush[bq * m_fs];
+      vl[i] = *(const int*)(m_len + bq * m_vs);
+      if constexpr (FUSED) ps[i] = *(const int*)(m_pos + bq * m_ps);
       if constexpr (SLOTS) sl[i] = *(const int*)(a.slot + bq * a.sl_s);
     }
     uint64_t fm[NO], zm[NO];  // flushing and other sequences
@@ -177,6 +183,16 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
       zm[i] = ~fm[i] & valid;
       nf += __popcll(fm[i]);
     }
+    // a few flushing sequences (as many as the grid has rows past the batch)
+    // get two workgroups each, for half of the vblocks (the rows then left
+    // over are spare: they take the last sequence's requests and end)
+    const int twice = nf < m_order ? nf : 0, y = blockIdx.y;
+    split = uni(y < 2 * twice) != 0;
+    half = uni(split ? y & 1 : 0);
+    int want = split ? y >> 1 : y - twice;
+    spare = uni(want >= a.B) != 0;
+    want = min(want, a.B - 1);
+    half = spare ? 1 : half;
     int at_f = 0, at_z = nf;
 #pragma unroll
     for (int i = 0; i < NO; ++i) {
@@ -184,7 +200,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
       const uint64_t below = (1ull << lane) - 1;
       const bool is_f = (fm[i] >> lane) & 1, is_z = (zm[i] >> lane) & 1;
       const int rank = is_f ? at_f + __popcll(fm[i] & below) : at_z + __popcll(zm[i] & below);
-      const uint64_t hit = __ballot((is_f || is_z) && rank == (int)blockIdx.y);
+      const uint64_t hit = __ballot((is_f || is_z) && rank == want);
       if (hit) {
         const int l = __builtin_ctzll(hit);
         b = 64 * i + l;
@@ -199,19 +215,19 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
     b = uni(b);
     if constexpr (!SLOTS) bs = b;
   } else {
-    n = (int)ld_u32_uniform(a.valid_len + b * a.vl_s);
-    if constexpr (FUSED) pos = (int)ld_u32_uniform(a.pos + b * a.pos_s);
+    n = (int)ld_u32_uniform(m_len + b * m_vs);
+    if constexpr (FUSED) pos = (int)ld_u32_uniform(m_pos + b * m_ps);
     if constexpr (SLOTS) bs = (int)ld_u32_uniform(a.slot + b * a.sl_s);
-    if (a.flush) {
-      const uintptr_t fa = (uintptr_t)(a.flush + b * a.fl_s);
+    if (m_flush) {
+      const uintptr_t fa = (uintptr_t)(m_flush + b * m_fs);
       const uint32_t word = ld_u32_uniform((const void*)(fa & ~(uintptr_t)3));
       do_flush = ((word >> (8u * (uint32_t)(fa & 3))) & 0xFFu) != 0;
     }
   }
   do_flush = uni(do_flush) != 0;
-  n = min(max(uni(n), 0), a.L);
+  n = min(max(uni(n), 0), m_L);
   pos = uni(pos);
-  if (pos < 0 || pos >= a.L) pos = -1;
+  if (pos < 0 || pos >= m_L) pos = -1;
   bs = uni(bs);
   if constexpr (SLOTS)
     if (bs < 0 || bs >= a.n_slots) bs = 0;
@@ -271,7 +287,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
         qw = act_bits(Act::round(qr.x / qd)) | (act_bits(Act::round(qr.y / qd)) << 16);
         const uint32_t kw = act_bits(Act::round(kr.x / kd)) | (act_bits(Act::round(kr.y / kd)) << 16);
         if (pos >= 0 && pos < n) *(uint32_t*)(lds + kLdsX + pos * kXS + 4 * lane) = kw;
-        if (grp == 0) {
+        if (grp == 0 && half == 0) {
           *(uint32_t*)(a.q_out + (b * a.qo_b + h * a.qo_h) + 4 * lane) = qw;
           if (pos >= 0) *(uint32_t*)(sbase(a.k, bs, a.k_b) + ((uint32_t)pos * a.k_t + h * a.k_h) + 4 * lane) = kw;
         }
@@ -320,7 +336,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
       const float sp = x <= 20.0f ? logf(1.0f + expf(x)) : x;  // kernel:560, as written there
       const float gate_new = Act::round(-expf(alog) * sp);
       const float beta_new = Act::round(1.0f / (1.0f + expf(-gate_value<GATE_F32>(ab1))));
-      if (pos >= 0 && lane == 0) {
+      if (pos >= 0 && lane == 0 && half == 0) {
         *(uint16_t*)(sbase(a.g, bs, a.g_b) + ((uint32_t)pos * a.g_t + hv * a.g_h)) = (uint16_t)act_bits(gate_new);
         *(uint16_t*)(sbase(a.beta, bs, a.be_b) + ((uint32_t)pos * a.be_t + hv * a.be_h)) = (uint16_t)act_bits(beta_new);
       }
@@ -334,6 +350,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
   constexpr int TPL = 64 / CPT;           // tokens per load
   constexpr int NVL = kMaxRing / TPL;     // loads per lane
 
+  if (spare) return;  // (here, not where it is found: the arguments' scalar loads would sink past it)
   if (!do_flush) {
     // ================= replay =====================================================
     u32x4_t cw[TPW][2];
@@ -537,7 +554,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
   // (the pair's v rows, one cache line a token and wave: they are read again,
   // tile by tile, from the cache)
   const uint32_t warm = ld32(v_rows + (uint32_t)(lane < n ? lane : 0) * a.v_t);
-  load_codes(0);
+  const int p0 = split ? half * (FV / 2) : 0, p1 = split ? p0 + FV / 2 : FV;  // the workgroup's vblocks
+  load_codes(p0);
   GDNR_COMPILER_FENCE();
   stage_x();
   asm volatile("" ::"v"(warm));
@@ -602,15 +620,15 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
   float* const red = (float*)(lds + kLdsZ + GW * (kRBytes + kFacBytes + kLamBytes));
   auto rebuild = [&](auto chunks) {
     constexpr int NF = decltype(chunks)::value;  // chunks (past the fill: zero keys, zero U~)
-    load_v(0);
     float sct[FV];
 #pragma unroll
     for (int p = 0; p < FV; ++p) sct[p] = f16_bits_to_f32(ld_u16_uniform(fs_rows + p * a.sc_v));
 #pragma unroll 1
-  for (int p = 0; p < FV; ++p) {
+  for (int p = p0; p < p1; ++p) {
     float scp = sct[0];
 #pragma unroll
     for (int k = 1; k < FV; ++k) scp = p == k ? sct[k] : scp;
+    load_v(p);
     // q[c] = X_c S^T, from S_0: on the codes, and on the query as a block of
     // its own
     f32x4_t q[NF], pq = {0.f, 0.f, 0.f, 0.f};
@@ -727,10 +745,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
       }
       u32x4_t k8[8];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
+      for (int g = 0; g < 2; ++g) {
         // (two groups' K^T operands at a time)
 #pragma unroll
-        for (int ct = 2 * g; ct < 2 * g + 2; ++ct) {
+        for (int ct = 4 * g; ct < 4 * g + 4; ++ct) {
           const uint2 k0 = kt_read(ko + 2 * NT * hh * kXS + 8 * ct);
           const uint2 k1 = kt_read(ko + (2 * hh + 1) * NT * kXS + 8 * ct);
           k8[ct] = u32x4_t{k0.x, k0.y, k1.x, k1.y};
@@ -738,7 +756,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
 #pragma unroll
         for (int d = 2; d >= 0; --d)
 #pragma unroll
-          for (int ct = 2 * g; ct < 2 * g + 2; ++ct) sv[ct] = mfma16(k8[ct], ub[d], sv[ct]);
+          for (int ct = 4 * g; ct < 4 * g + 4; ++ct) sv[ct] = mfma16(k8[ct], ub[d], sv[ct]);
         GDNR_COMPILER_FENCE();
       }
     }
@@ -747,10 +765,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
       for (int ct = 0; ct < 8; ++ct) sv[ct] *= down;
     }
     // (the next vblock's codes and v, while this one is requantised)
-    if (p + 1 < FV) {
-      load_codes(p + 1);
-      load_v(p + 1);
-    }
+    if (p + 1 < p1) load_codes(p + 1);
     // the reference quantiser (ref:36-37,83-99), as gdnr_decode.hip applies
     // it; the vblock's amax over the pair's two tiles through LDS (two slots
     // in turn: one barrier a vblock)
@@ -801,14 +816,17 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
     rebuild(std::integral_constant<int, NC>{});
   // the new token's v rows
   if constexpr (FUSED) {
-    if (pos >= 0 && lane < CPT) *(u32x4_t*)(v_rows + (uint32_t)pos * a.v_t + 16 * lane) = *(const g_u32x4*)(v_new + 16 * lane);
+    if (pos >= 0 && half == 0 && lane < CPT) *(u32x4_t*)(v_rows + (uint32_t)pos * a.v_t + 16 * lane) = *(const g_u32x4*)(v_new + 16 * lane);
   }
 }
 
 template <int VB, int WPH, bool FUSED, bool GATE_F32, bool SLOTS>
 int launch_variant(const StepArgs& a, hipStream_t s) {
-  const dim3 grid((unsigned)(a.H * a.units), (unsigned)a.B);
-  hipLaunchKernelGGL((ring_kernel<VB, WPH, FUSED, GATE_F32, SLOTS>), grid, dim3(64 * NW), ring_lds(NW / WPH, VB), s, a);
+  const int extra = a.seq_major ? std::min(a.B, kRingHalves) : 0;
+  const dim3 grid((unsigned)(a.H * a.units), (unsigned)(a.B + extra));
+  hipLaunchKernelGGL((ring_kernel<VB, WPH, FUSED, GATE_F32, SLOTS>), grid, dim3(64 * NW), ring_lds(NW / WPH, VB), s,
+                     a.valid_len, a.pos, a.flush, a.vl_s, a.pos_s, a.fl_s, a.L, a.units,
+                     a.seq_major ? 1 + extra : 0, a.G, a);
   return (int)hipGetLastError();
 }
 

@@ -43,10 +43,9 @@ SINGLE_SOURCES = ("gdnr_rmw", "gdnr_formats", "gdnr_status", "gdnr_probe")  # co
 # preloaded into SGPRs at wave launch (gfx950 kernarg preload), and its
 # wave-uniform branches (workgroup role, replay or flush) are left as scalar
 # branches rather than structurised into a chain in which one arm's values
-# stay live across the other; the ring kernel's (replay or flush) too
-SOURCE_FLAGS = {"gdnr_decode": ["-mllvm", "-amdgpu-kernarg-preload-count=13",
-                                "-mllvm", "-structurizecfg-skip-uniform-regions=true"],
-                "gdnr_ring": ["-mllvm", "-structurizecfg-skip-uniform-regions=true"]}
+# stay live across the other; the ring kernel likewise
+PRELOAD_UNIFORM = ["-mllvm", "-amdgpu-kernarg-preload-count=13", "-mllvm", "-structurizecfg-skip-uniform-regions=true"]
+SOURCE_FLAGS = {"gdnr_decode": PRELOAD_UNIFORM, "gdnr_ring": PRELOAD_UNIFORM}
 
 
 def _run(cmd: list[str], verbose: bool) -> None:

@@ -2,8 +2,8 @@
 17 to 64 tokens with 16-bit activations past the decode kernel's batches, at
 the sizes where its tiles end -- fills around every 16-token chunk, an empty
 ring and partial fills that flush, rings that end inside a chunk, each of its
-four workgroup shapes, and a launch of more than one round, whose flushing
-sequences are taken first -- against the fp64 oracle, and the fused launch
+four workgroup shapes, and launches of more than one round, whose flushing
+sequences are taken first (a few of them by two workgroups each) -- against the fp64 oracle, and the fused launch
 against prep then replay bit for bit.
 
 Tolerances: 16-bit outputs 2e-3 rel-L2 (bf16 rounds to 2^-9: 1.65e-3), codes
@@ -29,6 +29,7 @@ EDGES = [0, 1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64]
 # batch, heads, value heads, V, ring, dtype
 CASES = {
     "two heads a workgroup, two rounds": (50, 16, 32, 128, 64, torch.bfloat16),
+    "two rounds, full rings flushing in halves": (50, 16, 32, 128, 64, torch.bfloat16),
     "one head a workgroup": (17, 16, 32, 128, 33, torch.bfloat16),
     "odd group": (43, 4, 12, 128, 17, torch.bfloat16),
     "V=256": (13, 2, 4, 256, 40, torch.bfloat16),
@@ -43,7 +44,8 @@ def test_ring_kernel_edges(device, name):
     assert gdnr_lib.decode_plan(batch, heads, value_heads, value_dim, ring, act=dtype) is None
     fills = [min(f, ring) for f in EDGES] + [ring, ring - 1]
     valid = np.array([fills[i % len(fills)] for i in range(batch)])
-    flush = np.array([(i // len(fills) + i) % 2 == 0 or valid[i] == ring for i in range(batch)])
+    flush = np.array([("halves" not in name and (i // len(fills) + i) % 2 == 0) or valid[i] == ring
+                      for i in range(batch)])
     case = make_replay_case(batch, ring, device, seed=7, heads=heads, value_heads=value_heads, value_dim=value_dim,
                             dtype=dtype, warmup=8, valid=valid, flush=flush, reference_dist=True)
     block_v = min(128, value_dim)
