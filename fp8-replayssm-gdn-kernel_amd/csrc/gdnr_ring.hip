@@ -71,9 +71,10 @@ constexpr int kLdsZ = kLdsDq + 256;                      // replay or flush bloc
 // [64]; per wave the sums of c_t v_t f32 [32 VB]
 constexpr int kT0Bytes = 768, kCoefBytes = 256;
 // flush: per head R_c = (I + M_c)^-1 f32 [4][16][16] (M_c while it is
-// formed); per head (pre, post) f32 [64][2]; per head lam_c f32 [4]; the
+// formed); per head (pre, post) f32 [64][2]; per head lam_c f32 [4], the decay after
+// chunk c f32 [4] and lam f32; the
 // tiles' amax f32 [2][4]
-constexpr int kRBytes = NC * 1024, kFacBytes = kMaxRing * 8, kLamBytes = 16;
+constexpr int kRBytes = NC * 1024, kFacBytes = kMaxRing * 8, kLamBytes = 48;
 
 constexpr int ring_lds(int gw, int vb) {
   const int replay = gw * (kT0Bytes + kCoefBytes) + NW * 32 * vb * 4, flush = gw * (kRBytes + kFacBytes + kLamBytes) + 2 * NW * 4;
@@ -120,6 +121,27 @@ __device__ __forceinline__ Split3 split3_act(float x, float y) {
 // 32 (l16 >> 2) + 4 ct + (l16 & 3) of the four rows
 __device__ __forceinline__ uint2 kt_read(int off) {
   return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(ring_smem + off)));
+}
+// double-precision decays of a flush: DPP moves and products over a 16-lane row
+template <int CTRL>
+__device__ __forceinline__ double dpp_row64(double x, double fill) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, x), f = __builtin_bit_cast(uint64_t, fill);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp((int)(uint32_t)f, (int)(uint32_t)b, CTRL, 0xF, 0xF, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp((int)(f >> 32), (int)(b >> 32), CTRL, 0xF, 0xF, false);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+// every lane of each 16-lane row gets lane n of its row
+__device__ __forceinline__ double row_bcast64(double x, int n) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = __float_as_uint(row_bcast_n(__uint_as_float((uint32_t)b), n));
+  const uint32_t hi = __float_as_uint(row_bcast_n(__uint_as_float((uint32_t)(b >> 32)), n));
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ double rdl64(double x, int lane) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 __device__ __forceinline__ void lds_barrier() {
   GDNR_WAIT_LGKM0();
@@ -326,11 +348,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
       if (l16 == 0) *(f32x4_t*)(lds + kLdsDq + 4 * (NT * c + 4 * q4)) = d;
     }
   };
-  // lane t: gamma and beta of token t (1 and 0 at or past the fill), the new
+  // lane t: the log decay g and beta (0 at or past the fill) of token t, the new
   // token's from the preparation formulas (kernel:534-562) and appended
   const bool on = lane < n;
-  auto gates = [&](float& gam, float& bet) {
-    float gg = act_val(g_raw), bb = act_val(be_raw);
+  auto gates = [&](float& gg, float& bet) {
+    gg = act_val(g_raw);
+    float bb = act_val(be_raw);
     if constexpr (FUSED) {
       const float x = gate_value<GATE_F32>(ab0) + dtb;
       const float sp = x <= 20.0f ? logf(1.0f + expf(x)) : x;  // kernel:560, as written there
@@ -343,7 +366,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
       gg = lane == pos ? gate_new : gg;
       bb = lane == pos ? beta_new : bb;
     }
-    gam = on ? expf(gg) : 1.f;
     bet = on ? bb : 0.f;
   };
   constexpr int CPT = RPW * ES / 16;      // 16-byte pieces of a token's v rows of the wave
@@ -387,8 +409,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
     if (part == 0) {
       // the head's coefficient chain (lane t: token t), as the chunked chain
       // of gdnr_decode.hip runs it
-      float gam, bet;
-      gates(gam, bet);
+      float gg, bet;
+      gates(gg, bet);
+      const float gam = on ? expf(gg) : 1.f;
       const float suf_in = row_suffix_prod(gam);
       const float suf_ex = dpp_row<0x101>(suf_in, 1.f);
       const float lamc = row_bcast<0>(suf_in);
@@ -570,13 +593,27 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
     // prod_{x<=t} gamma_x, post_t = beta_t prod_{x>t} gamma_x, lam_c,
     // M[t][s] = beta_s prod_{s<x<=t} gamma_x G[s][t] (s < t) and
     // R = (I + M)^-1 by forward substitution, lane = column
-    float gam, bet;
-    gates(gam, bet);
-    const float suf_in = row_suffix_prod(gam);
-    const float suf_ex = dpp_row<0x101>(suf_in, 1.f);
-    const float pre = row_prefix_prod(gam);
-    *(float2*)(fl + 8 * lane) = make_float2(pre, bet * suf_ex);
-    if (l16 == 0) ll[q4] = suf_in;
+    // (the decays in double: f32 products of up to 64 gammas cost a quarter of
+    // the rounding that shows in the codes, 5.3e-6 of them against 3.9e-6 a
+    // rounding off the exact state's; 1 us of a 25 us launch of 24 flushes)
+    float gg, bet;
+    gates(gg, bet);
+    const double gam = on ? exp((double)gg) : 1.0;
+    double pre = gam, suf_in = gam;
+    pre *= dpp_row64<0x111>(pre, 1.0), suf_in *= dpp_row64<0x101>(suf_in, 1.0);
+    pre *= dpp_row64<0x112>(pre, 1.0), suf_in *= dpp_row64<0x102>(suf_in, 1.0);
+    pre *= dpp_row64<0x114>(pre, 1.0), suf_in *= dpp_row64<0x104>(suf_in, 1.0);
+    pre *= dpp_row64<0x118>(pre, 1.0), suf_in *= dpp_row64<0x108>(suf_in, 1.0);
+    const double suf_ex = dpp_row64<0x101>(suf_in, 1.0);
+    *(float2*)(fl + 8 * lane) = make_float2((float)pre, (float)((double)bet * suf_ex));
+    // lam_c, and the decay from chunk c's end to the ring's (lane 16 c); [8]: lam
+    const double l1 = rdl64(suf_in, NT), l2 = rdl64(suf_in, 2 * NT), l3 = rdl64(suf_in, 3 * NT);
+    const double after = q4 == 0 ? l1 * l2 * l3 : q4 == 1 ? l2 * l3 : q4 == 2 ? l3 : 1.0;
+    if (l16 == 0) {
+      ll[q4] = (float)suf_in;
+      ll[4 + q4] = (float)after;
+      if (q4 == 0) ll[8] = (float)(suf_in * after);
+    }
     const int nc = min(max(n - NT * q4, 0), NT);
     float gcol[NT];
     {
@@ -589,12 +626,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
     }
     float* Mm = (float*)rl + q4 * 256;
     {
-      float run = 1.f;
+      double run = bet;
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const float gt = row_bcast_n(gam, t);
+      for (int t = 1; t < NT; ++t) {
+        const double gt = row_bcast64(gam, t);  // (in every lane: the moves read the whole row)
         run = t > l16 ? run * gt : run;
-        Mm[t * NT + l16] = (l16 < t && t < nc) ? bet * run * gcol[t] : 0.f;
+        Mm[t * NT + l16] = (l16 < t && t < nc) ? (float)(run * (double)gcol[t]) : 0.f;
       }
     }
     float rc[NT];
@@ -645,7 +682,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
     int t0 = 4 * q4;
     asm volatile("" : "+v"(t0));            // (the 16 tokens are compared as they come up)
     float o = q4 == 0 ? scp * pq[0] : 0.f;  // (S_0 q at every q4: counted once)
-    float lcs[NF];
 #pragma unroll
     for (int c = 0; c < NF; ++c) q[c] *= scp;
     // chunk by chunk: U~_c from q[c], then q of every later chunk taken to
@@ -658,7 +694,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
       const f32x4_t rr = *(const f32x4_t*)(rl + 1024 * c + 4 * (l16 * NT + 4 * q4));
       const f32x4_t dq = *(const f32x4_t*)(lds + kLdsDq + 4 * (NT * c + 4 * q4));
       const float lc = ll[c];
-      lcs[c] = lc;
       float we[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e)
@@ -694,13 +729,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
       }
     }
     // U~ decayed to the end of the ring, and the checkpoint's own weight
-    float lam = 1.f;
 #pragma unroll
-    for (int c = NF - 1; c >= 0; --c) {
-      if (c < NF - 1) q[c] *= lam;
-      lam *= lcs[c];
-    }
-    lam *= scp;
+    for (int c = 0; c < NF - 1; ++c) q[c] *= ll[4 + c];
+    const float lam = ll[8] * scp;
     GDNR_COMPILER_FENCE();
     // the f16 parts of a row's U~ scaled by a power of two (the row's largest
     // to [2^13, 2^14)), undone on the row's state
