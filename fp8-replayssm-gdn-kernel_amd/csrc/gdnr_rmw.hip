@@ -18,14 +18,19 @@
 // together -- equal to the reference's sum of (S q) up to fp32 rounding.
 //
 // HBM-bound: every state byte is read once and written once; nothing else is
-// larger than a row. A wave owns 32 V-rows of one value head; a lane owns one
+// larger than a row. A wave owns RPW V-rows of one value head; a lane owns one
 // 16-byte chunk of a row (8 elements of a 2-byte state, 4 of an f32 one), so
 // a row spans 16 or 32 lanes and each wave instruction moves 4 or 2 whole
 // rows. All of a wave's chunk loads are issued before the first is used; each
 // row's store follows its compute while later rows are still arriving. The
 // row sums reduce across the row's lanes with DPP (plus one swizzle for
-// 32-lane rows). Measured on MI355X at the C1 shape: within 15% of an in-place
-// load/store kernel with the same access pattern and no arithmetic.
+// 32-lane rows). Loads and stores are non-temporal: a layer's state is next
+// touched a whole step later, after every other layer's. Measured on MI355X
+// (us a step of a bf16 state, HV=32, V=128, rotating states past the Infinity
+// Cache; before: plain accesses, 32 rows a wave): B=64 25.1 (33.0), B=32 12.5
+// (18.6), B=8 5.5 (8.2), B=1 3.8 (5.3); f32 B=64 49.4 (61.2), B=16 12.0 (17.7).
+// 5.3 TB/s read + written at B=64. A state that stays in that cache from step
+// to step (one layer alone) gains nothing or loses some: B=64 22.9 (22.6).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -78,7 +83,7 @@ __device__ __forceinline__ u32x4_t f32_to_chunk(const float* f) {
   }
 }
 
-// RPW V-rows of one value head per wave, four waves per workgroup over
+// RPW V-rows of one value head per wave (launch_rows), four waves per workgroup over
 // consecutive rows of a sequence's [HV, V] row space. PACKED: the production
 // contract -- q, k, v from the raw mixed_qkv row, q and k L2-normalised and
 // the gates formed in fp32 here (the formulas of the full-contract prep,
@@ -109,7 +114,7 @@ __global__ __launch_bounds__(256) void rmw_step_kernel(const RmwArgs a) {
   const uint32_t lane_off = (uint32_t)rsub * row_bytes + 16u * (uint32_t)cl;
   u32x4_t ch[NI];
 #pragma unroll
-  for (int i = 0; i < NI; ++i) ch[i] = *(const u32x4_t*)(sbase + (lane_off + (uint32_t)(i * RPI) * row_bytes));
+  for (int i = 0; i < NI; ++i) ch[i] = __builtin_nontemporal_load((const u32x4_t*)(sbase + (lane_off + (uint32_t)(i * RPI) * row_bytes)));
 
   // k and q of the key head at this lane's columns, the head's gate and
   // beta, and the v element of each row this lane touches
@@ -176,16 +181,32 @@ __global__ __launch_bounds__(256) void rmw_step_kernel(const RmwArgs a) {
 #pragma unroll
     for (int e = 0; e < EPC; ++e) s[e] = fmaf(c, kf[e], s[e]);
     const float o = fmaf(c, kq, sq);
-    *(u32x4_t*)(sbase + (lane_off + (uint32_t)(i * RPI) * row_bytes)) = f32_to_chunk<S>(s);
+    __builtin_nontemporal_store(f32_to_chunk<S>(s), (u32x4_t*)(sbase + (lane_off + (uint32_t)(i * RPI) * row_bytes)));
     if (cl == 0) Act::st(op, i * RPI, o * a.out_scale);
   }
 }
 
+template <class S, class Act, int RPW, bool PACKED, bool GATE_F32>
+void launch_height(const RmwArgs& a, hipStream_t s) {
+  const int rows = a.HV * a.V;
+  const dim3 grid((rows + 4 * RPW - 1) / (4 * RPW), a.B);
+  hipLaunchKernelGGL((rmw_step_kernel<S, Act, RPW, PACKED, GATE_F32>), grid, dim3(256), 0, s, a);
+}
+
+// Rows per wave (a divisor of V: a wave's rows stay in one head): 4 KiB of a
+// row block, so that a small batch covers the chip; 16 KiB of a 2-byte state
+// once that leaves at least three workgroups per compute unit (us at 64 and 16
+// rows: B=32 15.0 and 12.5, B=48 19.8 and 20.6, B=64 25.1 and 27.3, B=128 53.0
+// and 51.9 to 54.3; an f32 state at 32 and 8 rows: B=64 51.7 and 49.4).
 template <class S, class Act, bool PACKED = false, bool GATE_F32 = false>
 void launch_rows(const RmwArgs& a, hipStream_t s) {
-  const int rows = a.HV * a.V;  // V % 32 == 0: a wave's rows stay in one head
-  const dim3 grid((rows + 4 * 32 - 1) / (4 * 32), a.B);
-  hipLaunchKernelGGL((rmw_step_kernel<S, Act, 32, PACKED, GATE_F32>), grid, dim3(256), 0, s, a);
+  if constexpr (S::kBytes == 4) {
+    launch_height<S, Act, 8, PACKED, GATE_F32>(a, s);
+  } else if (a.V % 64 == 0 && (int64_t)a.B * a.HV * a.V >= 3 * 256 * (int64_t)device_cus()) {
+    launch_height<S, Act, 64, PACKED, GATE_F32>(a, s);
+  } else {
+    launch_height<S, Act, 16, PACKED, GATE_F32>(a, s);
+  }
 }
 
 template <class S>
