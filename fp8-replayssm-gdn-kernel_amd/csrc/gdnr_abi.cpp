@@ -546,6 +546,8 @@ void fit_decode(gdnr::ReplayArgs* a) {
       break;
     }
   }
+  // (of many rounds: late flushes change places with early replays)
+  if (large && a->flush) a->seq_major |= 2;
   // vblocks per row wave: V / 32 / nwh
   a->lds_bytes = gdnr::decode_lds_bytes(a->units, a->gw * a->nwh, a->V / 32 / a->nwh, 1);
 }

@@ -214,7 +214,7 @@ __host__ __device__ constexpr int unit_lds(int nch, int rpu, int vb) {
 // (gfx950 kernarg preload, the build's -amdgpu-kernarg-preload-count): the
 // first requests of every wave issue before any scalar load returns.
 // Everything else comes from the StepArgs block.
-template <int TPW, int NWH, int NCH, bool FUSED, bool GATE_F32, bool SLOTS>
+template <int TPW, int NWH, int NCH, bool FUSED, bool GATE_F32, bool SLOTS, bool SWAP>
 __global__ __launch_bounds__(768) __attribute__((amdgpu_waves_per_eu(3))) void decode_kernel(
     uint8_t* ckpt, uint8_t* kring, uint32_t ck_b, uint32_t ck_h, uint32_t ck_v, uint32_t k_b, uint32_t k_t,
     uint32_t k_h, int32_t L, int32_t G, int32_t shape, const StepArgs a) {
@@ -252,7 +252,25 @@ __global__ __launch_bounds__(768) __attribute__((amdgpu_waves_per_eu(3))) void d
   const int uh = HP == 2 ? (u & 1) : 0, us = HP == 2 ? (u >> 1) : u;
   const int r = uni(bx * HP + uh);  // the unit's (key head, value-head group)
   const int n_grp = uni(G / gw);
-  const int h = uni(r / n_grp), grp = r - h * n_grp, b0 = uni(by * SP + us);
+  const int h = uni(r / n_grp), grp = r - h * n_grp;
+  int b0 = uni(by * SP + us);
+  // SWAP (launches of many rounds of workgroups, one unit each): sequences b
+  // and B - 1 - b change places when only the later one flushes. A flush runs
+  // several times as long as a replay; one that starts in the launch's last
+  // rounds ends it late (B=512, L=8, 64 flushes spread over the batch 79.3 us,
+  // so 70.2; B=256, L=16, 16 of them 41.4 and 36.5; no flush at all 61.6 and
+  // 62.2). An instantiation of its own: the flags' loads in the others' prologue
+  // cost them 1 to 3%.
+  if constexpr (SWAP) {
+    const int other = a.B - 1 - b0;
+    auto flushes = [&](int bq) {
+      const uintptr_t fa = (uintptr_t)(a.flush + (uint32_t)bq * a.fl_s);
+      const uint32_t word = ld_u32_uniform((const void*)(fa & ~(uintptr_t)3));
+      return uni((int)((word >> (8u * (uint32_t)(fa & 3))) & 0xFFu)) != 0;
+    };
+    const bool late = flushes(max(b0, other)), early = flushes(min(b0, other));
+    b0 = late && !early ? other : b0;
+  }
   const int hv0 = h * G + grp * gw;              // first value head of the unit
   uint8_t* const ul = lds + u * unit_lds(NCH, rpu, TPW / 2);  // the unit's LDS block
 
@@ -1589,30 +1607,39 @@ __global__ __launch_bounds__(768) __attribute__((amdgpu_waves_per_eu(3))) void d
   }
 }
 
-template <int TPW, int NWH, int NCH, bool FUSED, bool GATE_F32, bool SLOTS>
+template <int TPW, int NWH, int NCH, bool FUSED, bool GATE_F32, bool SLOTS, bool SWAP>
 int launch_variant(const StepArgs& a, hipStream_t s) {
   const int hp = a.units == 4 ? 2 : 1, sp = a.units / hp;  // as in the kernel
   const unsigned gh = (unsigned)(a.H * (a.G / a.gw) / hp), gs = (unsigned)(a.B / sp);
-  const dim3 grid(a.seq_major ? gs : gh, a.seq_major ? gh : gs),
+  const bool seq_major = (a.seq_major & 1) != 0;
+  const dim3 grid(seq_major ? gs : gh, seq_major ? gh : gs),
       block((unsigned)(64 * a.units * (1 + a.gw * NWH)));
-  auto kernel = decode_kernel<TPW, NWH, NCH, FUSED, GATE_F32, SLOTS>;
+  auto kernel = decode_kernel<TPW, NWH, NCH, FUSED, GATE_F32, SLOTS, SWAP>;
   if (a.lds_bytes > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, a.lds_bytes);
     if (e != hipSuccess) return (int)e;
   }
   hipLaunchKernelGGL(kernel, grid, block, a.lds_bytes, s, a.ckpt, a.k, a.ck_b, a.ck_h, a.ck_v, a.k_b, a.k_t, a.k_h,
-                     a.L, a.G, a.gw | (a.units << 8) | (a.seq_major << 16), a);
+                     a.L, a.G, a.gw | (a.units << 8) | ((seq_major ? 1 : 0) << 16), a);
   return 0;
 }
 
-template <int TPW, int NWH, int NCH = 1>
+template <int TPW, int NWH, int NCH, bool SWAP>
+int launch_modes(const StepArgs& a, bool fused, bool gate_f32, hipStream_t s) {
+  if (!fused) return launch_variant<TPW, NWH, NCH, false, false, false, SWAP>(a, s);
+  if (a.slot && gate_f32) return launch_variant<TPW, NWH, NCH, true, true, true, SWAP>(a, s);
+  if (a.slot) return launch_variant<TPW, NWH, NCH, true, false, true, SWAP>(a, s);
+  if (gate_f32) return launch_variant<TPW, NWH, NCH, true, true, false, SWAP>(a, s);
+  return launch_variant<TPW, NWH, NCH, true, false, false, SWAP>(a, s);
+}
+
+// MANY: a plan that launches of many rounds take (fit_decode)
+template <int TPW, int NWH, int NCH = 1, bool MANY = false>
 int launch_shape(const StepArgs& a, bool fused, bool gate_f32, hipStream_t s) {
-  if (!fused) return launch_variant<TPW, NWH, NCH, false, false, false>(a, s);
-  if (a.slot && gate_f32) return launch_variant<TPW, NWH, NCH, true, true, true>(a, s);
-  if (a.slot) return launch_variant<TPW, NWH, NCH, true, false, true>(a, s);
-  if (gate_f32) return launch_variant<TPW, NWH, NCH, true, true, false>(a, s);
-  return launch_variant<TPW, NWH, NCH, true, false, false>(a, s);
+  if constexpr (MANY)
+    if (a.seq_major & 2) return launch_modes<TPW, NWH, NCH, true>(a, fused, gate_f32, s);
+  return launch_modes<TPW, NWH, NCH, false>(a, fused, gate_f32, s);
 }
 
 }  // namespace
@@ -1638,10 +1665,10 @@ int GDNR_SUFFIX(launch_decode)(const StepArgs& a, bool fused, bool gate_f32, voi
   else if (a.L > kStepRing)
     rc = a.sw == 1 ? launch_shape<4, 1, kDecodeChunks>(a, fused, gate_f32, s)
                    : launch_shape<4, 2, kDecodeChunks>(a, fused, gate_f32, s);
-  else if (a.sw == 1) rc = launch_shape<4, 1>(a, fused, gate_f32, s);
+  else if (a.sw == 1) rc = launch_shape<4, 1, 1, true>(a, fused, gate_f32, s);
   else if (a.sw == 2 && a.nwh == 4) rc = launch_shape<2, 4>(a, fused, gate_f32, s);
-  else if (a.sw == 2) rc = launch_shape<8, 1>(a, fused, gate_f32, s);
-  else rc = launch_shape<8, 2>(a, fused, gate_f32, s);
+  else if (a.sw == 2) rc = launch_shape<8, 1, 1, true>(a, fused, gate_f32, s);
+  else rc = launch_shape<8, 2, 1, true>(a, fused, gate_f32, s);
   if (rc) return rc;
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : (int)e;

@@ -59,7 +59,10 @@ struct ReplayArgs {
   int32_t sw, rpw, lds_knew, lds_flag, lds_c, lds_g;
   int32_t units;  // decode kernel: (key head, value-head group) units per workgroup
   int32_t nwh;    // decode kernel: row waves per value head
-  int32_t seq_major;  // decode kernel: workgroups numbered sequence-fastest (grid x = sequences)
+  // decode kernel: bit 0: workgroups numbered sequence-fastest (grid x =
+  // sequences), bit 1: late flushes change places with early replays; ring
+  // kernel: flushing sequences first
+  int32_t seq_major;
   // flush (MFMA rebuild), per head: R = (I + M)^-1 [16 x 16] f32, per-token
   // factors (pre, post, dq, -) f32, lam_all f32; K^T operand tiles [K x 16]
   // in the ring dtype; per-head scratch (3 KiB)
