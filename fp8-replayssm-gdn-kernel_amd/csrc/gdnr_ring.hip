@@ -661,185 +661,185 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
 #pragma unroll
     for (int p = 0; p < FV; ++p) sct[p] = f16_bits_to_f32(ld_u16_uniform(fs_rows + p * a.sc_v));
 #pragma unroll 1
-  for (int p = p0; p < p1; ++p) {
-    float scp = sct[0];
+    for (int p = p0; p < p1; ++p) {
+      float scp = sct[0];
 #pragma unroll
-    for (int k = 1; k < FV; ++k) scp = p == k ? sct[k] : scp;
-    load_v(p);
-    // q[c] = X_c S^T, from S_0: on the codes, and on the query as a block of
-    // its own
-    f32x4_t q[NF], pq = {0.f, 0.f, 0.f, 0.f};
+      for (int k = 1; k < FV; ++k) scp = p == k ? sct[k] : scp;
+      load_v(p);
+      // q[c] = X_c S^T, from S_0: on the codes, and on the query as a block of
+      // its own
+      f32x4_t q[NF], pq = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int c = 0; c < NF; ++c) q[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int c = 0; c < NF; ++c) q[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const u32x4_t bv = codes8(cw, m);
-      pq = mfma16(q_op(m), bv, pq);
+      for (int m = 0; m < 4; ++m) {
+        const u32x4_t bv = codes8(cw, m);
+        pq = mfma16(q_op(m), bv, pq);
 #pragma unroll
-      for (int c = 0; c < NF; ++c) q[c] = mfma16(x_op(c, m), bv, q[c]);
-      if (m & 1) GDNR_COMPILER_FENCE();
-    }
-    int t0 = 4 * q4;
-    asm volatile("" : "+v"(t0));            // (the 16 tokens are compared as they come up)
-    float o = q4 == 0 ? scp * pq[0] : 0.f;  // (S_0 q at every q4: counted once)
+        for (int c = 0; c < NF; ++c) q[c] = mfma16(x_op(c, m), bv, q[c]);
+        if (m & 1) GDNR_COMPILER_FENCE();
+      }
+      int t0 = 4 * q4;
+      asm volatile("" : "+v"(t0));            // (the 16 tokens are compared as they come up)
+      float o = q4 == 0 ? scp * pq[0] : 0.f;  // (S_0 q at every q4: counted once)
 #pragma unroll
-    for (int c = 0; c < NF; ++c) q[c] *= scp;
-    // chunk by chunk: U~_c from q[c], then q of every later chunk taken to
-    // the state after chunk c (two accumulators where the next step waits)
+      for (int c = 0; c < NF; ++c) q[c] *= scp;
+      // chunk by chunk: U~_c from q[c], then q of every later chunk taken to
+      // the state after chunk c (two accumulators where the next step waits)
 #pragma unroll
-    for (int c = 0; c < NF; ++c) {
-      const f32x4_t f01 = *(const f32x4_t*)(fl + 8 * (NT * c + 4 * q4));
-      const f32x4_t f23 = *(const f32x4_t*)(fl + 8 * (NT * c + 4 * q4) + 16);
-      const float pre[4] = {f01[0], f01[2], f23[0], f23[2]}, post[4] = {f01[1], f01[3], f23[1], f23[3]};
-      const f32x4_t rr = *(const f32x4_t*)(rl + 1024 * c + 4 * (l16 * NT + 4 * q4));
-      const f32x4_t dq = *(const f32x4_t*)(lds + kLdsDq + 4 * (NT * c + 4 * q4));
-      const float lc = ll[c];
-      float we[4];
+      for (int c = 0; c < NF; ++c) {
+        const f32x4_t f01 = *(const f32x4_t*)(fl + 8 * (NT * c + 4 * q4));
+        const f32x4_t f23 = *(const f32x4_t*)(fl + 8 * (NT * c + 4 * q4) + 16);
+        const float pre[4] = {f01[0], f01[2], f23[0], f23[2]}, post[4] = {f01[1], f01[3], f23[1], f23[3]};
+        const f32x4_t rr = *(const f32x4_t*)(rl + 1024 * c + 4 * (l16 * NT + 4 * q4));
+        const f32x4_t dq = *(const f32x4_t*)(lds + kLdsDq + 4 * (NT * c + 4 * q4));
+        const float lc = ll[c];
+        float we[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        we[e] = fmaf(-pre[e], q[c][e], act_val(e & 1 ? vw[c][e >> 1] >> 16 : vw[c][e >> 1]));
-      if ((FUSED && c == pos / NT) || NT * (c + 1) > n) {  // (the new token's chunk, the fill's end)
+        for (int e = 0; e < 4; ++e)
+          we[e] = fmaf(-pre[e], q[c][e], act_val(e & 1 ? vw[c][e >> 1] >> 16 : vw[c][e >> 1]));
+        if ((FUSED && c == pos / NT) || NT * (c + 1) > n) {  // (the new token's chunk, the fill's end)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int t = t0 + NT * c + e;
+            if (FUSED && t == pos) we[e] = fmaf(-pre[e], q[c][e], act_val(vwn));
+            we[e] = t < n ? we[e] : 0.f;
+          }
+        }
+        f32x4_t ua = {0.f, 0.f, 0.f, 0.f}, ub = ua;
+        ua = __builtin_amdgcn_mfma_f32_16x16x4f32(rr[0], we[0], ua, 0, 0, 0);
+        ub = __builtin_amdgcn_mfma_f32_16x16x4f32(rr[1], we[1], ub, 0, 0, 0);
+        ua = __builtin_amdgcn_mfma_f32_16x16x4f32(rr[2], we[2], ua, 0, 0, 0);
+        ub = __builtin_amdgcn_mfma_f32_16x16x4f32(rr[3], we[3], ub, 0, 0, 0);
+        o *= lc;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int t = t0 + NT * c + e;
-          if (FUSED && t == pos) we[e] = fmaf(-pre[e], q[c][e], act_val(vwn));
-          we[e] = t < n ? we[e] : 0.f;
-        }
-      }
-      f32x4_t ua = {0.f, 0.f, 0.f, 0.f}, ub = ua;
-      ua = __builtin_amdgcn_mfma_f32_16x16x4f32(rr[0], we[0], ua, 0, 0, 0);
-      ub = __builtin_amdgcn_mfma_f32_16x16x4f32(rr[1], we[1], ub, 0, 0, 0);
-      ua = __builtin_amdgcn_mfma_f32_16x16x4f32(rr[2], we[2], ua, 0, 0, 0);
-      ub = __builtin_amdgcn_mfma_f32_16x16x4f32(rr[3], we[3], ub, 0, 0, 0);
-      o *= lc;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        q[c][e] = (ua[e] + ub[e]) * post[e];
-        o = fmaf(q[c][e], dq[e], o);
-      }
-#pragma unroll
-      for (int cc = c + 1; cc < NF; ++cc) {
-        const f32x4_t g4 = *(const f32x4_t*)(lds + gram_tile(c, cc) + 4 * (l16 * kGS + 4 * q4));
-        f32x4_t qa = q[cc] * lc, qb = {0.f, 0.f, 0.f, 0.f};
-        qa = __builtin_amdgcn_mfma_f32_16x16x4f32(g4[0], q[c][0], qa, 0, 0, 0);
-        qb = __builtin_amdgcn_mfma_f32_16x16x4f32(g4[1], q[c][1], qb, 0, 0, 0);
-        qa = __builtin_amdgcn_mfma_f32_16x16x4f32(g4[2], q[c][2], qa, 0, 0, 0);
-        qb = __builtin_amdgcn_mfma_f32_16x16x4f32(g4[3], q[c][3], qb, 0, 0, 0);
-        q[cc] = qa + qb;
-      }
-    }
-    // U~ decayed to the end of the ring, and the checkpoint's own weight
-#pragma unroll
-    for (int c = 0; c < NF - 1; ++c) q[c] *= ll[4 + c];
-    const float lam = ll[8] * scp;
-    GDNR_COMPILER_FENCE();
-    // the f16 parts of a row's U~ scaled by a power of two (the row's largest
-    // to [2^13, 2^14)), undone on the row's state
-    float up = 1.f, down = 1.f;
-    if constexpr (!kBF16) {
-      float mx = 0.f;
-#pragma unroll
-      for (int c = 0; c < NF; ++c)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) mx = fmaxf(mx, fabsf(q[c][e]));
-      mx = fmaxf(mx, __shfl_xor(mx, 16));
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
-      if (mx > 0x1p-80f && mx < 0x1p80f) {
-        int ex;
-        (void)frexpf(mx, &ex);
-        up = ldexpf(1.f, 14 - ex);
-        down = ldexpf(1.f, ex - 14);
-      }
-    }
-    // S_n of the tile's 8 column groups: lane (nn, q4) gets
-    // S_n[row][32 q4 + 4 ct + e], code byte 4 ct + e of its 32; U~ of two
-    // chunks at a time in three parts
-    const float ls = lam * up;
-    const int ko = kLdsX + (4 * q4 + (l16 >> 2)) * kXS + 64 * (l16 & 3);
-    f32x4_t sv[8];
-#pragma unroll
-    for (int ct = 0; ct < 8; ++ct) {
-      float f[4];
-      fp8x4_to_f32(cw[ct >> 2][ct & 3], f);
-      sv[ct] = f32x4_t{ls * f[0], ls * f[1], ls * f[2], ls * f[3]};
-    }
-#pragma unroll
-    for (int hh = 0; hh < NF / 2; ++hh) {
-      u32x4_t ub[3];
-#pragma unroll
-      for (int d = 0; d < 2; ++d) {
-        const f32x4_t x = q[2 * hh + d] * up;
-        const Split3 s01 = split3_act(x[0], x[1]), s23 = split3_act(x[2], x[3]);
-        ub[0][2 * d] = s01.hi, ub[0][2 * d + 1] = s23.hi;
-        ub[1][2 * d] = s01.mid, ub[1][2 * d + 1] = s23.mid;
-        ub[2][2 * d] = s01.lo, ub[2][2 * d + 1] = s23.lo;
-      }
-      u32x4_t k8[8];
-#pragma unroll
-      for (int g = 0; g < 2; ++g) {
-        // (two groups' K^T operands at a time)
-#pragma unroll
-        for (int ct = 4 * g; ct < 4 * g + 4; ++ct) {
-          const uint2 k0 = kt_read(ko + 2 * NT * hh * kXS + 8 * ct);
-          const uint2 k1 = kt_read(ko + (2 * hh + 1) * NT * kXS + 8 * ct);
-          k8[ct] = u32x4_t{k0.x, k0.y, k1.x, k1.y};
+          q[c][e] = (ua[e] + ub[e]) * post[e];
+          o = fmaf(q[c][e], dq[e], o);
         }
 #pragma unroll
-        for (int d = 2; d >= 0; --d)
-#pragma unroll
-          for (int ct = 4 * g; ct < 4 * g + 4; ++ct) sv[ct] = mfma16(k8[ct], ub[d], sv[ct]);
-        GDNR_COMPILER_FENCE();
+        for (int cc = c + 1; cc < NF; ++cc) {
+          const f32x4_t g4 = *(const f32x4_t*)(lds + gram_tile(c, cc) + 4 * (l16 * kGS + 4 * q4));
+          f32x4_t qa = q[cc] * lc, qb = {0.f, 0.f, 0.f, 0.f};
+          qa = __builtin_amdgcn_mfma_f32_16x16x4f32(g4[0], q[c][0], qa, 0, 0, 0);
+          qb = __builtin_amdgcn_mfma_f32_16x16x4f32(g4[1], q[c][1], qb, 0, 0, 0);
+          qa = __builtin_amdgcn_mfma_f32_16x16x4f32(g4[2], q[c][2], qa, 0, 0, 0);
+          qb = __builtin_amdgcn_mfma_f32_16x16x4f32(g4[3], q[c][3], qb, 0, 0, 0);
+          q[cc] = qa + qb;
+        }
       }
-    }
-    if constexpr (!kBF16) {
+      // U~ decayed to the end of the ring, and the checkpoint's own weight
 #pragma unroll
-      for (int ct = 0; ct < 8; ++ct) sv[ct] *= down;
-    }
-    // (the next vblock's codes and v, while this one is requantised)
-    if (p + 1 < p1) load_codes(p + 1);
-    // the reference quantiser (ref:36-37,83-99), as gdnr_decode.hip applies
-    // it; the vblock's amax over the pair's two tiles through LDS (two slots
-    // in turn: one barrier a vblock)
-    float am = 0.f, am1 = 0.f;
+      for (int c = 0; c < NF - 1; ++c) q[c] *= ll[4 + c];
+      const float lam = ll[8] * scp;
+      GDNR_COMPILER_FENCE();
+      // the f16 parts of a row's U~ scaled by a power of two (the row's largest
+      // to [2^13, 2^14)), undone on the row's state
+      float up = 1.f, down = 1.f;
+      if constexpr (!kBF16) {
+        float mx = 0.f;
 #pragma unroll
-    for (int ct = 0; ct < 8; ++ct) {
-      am = max3_abs(am, sv[ct][0], sv[ct][1]);
-      am1 = max3_abs(am1, sv[ct][2], sv[ct][3]);
-    }
-    const float am_mine = __uint_as_float(wave_max_u32(__float_as_uint(__builtin_elementwise_maximum(am, am1))));
-    float* const rp = red + NW * (p & 1);
-    if (lane == 0) rp[w] = am_mine;
-    lds_barrier();
-    const uint32_t am_bits = (uint32_t)uni((int)max(__float_as_uint(am_mine), __float_as_uint(rp[w ^ 1])));
-    const float amax = __uint_as_float(am_bits);
-    const float s32 = (amax > 0.0f) ? amax / 448.0f : 1.0f;
-    {
-      o = rows_reduce_scatter(o, 0.f, 0.f, 0.f);
-      if (q4 == 0) Act::st(fo_rows, 32 * p + l16, o * a.out_scale);
-    }
-    uint8_t* const row = fc_rows + (uint32_t)(32 * p + l16) * a.ck_v + 32 * q4;
-    auto store_codes = [&](auto quant) {
+        for (int c = 0; c < NF; ++c)
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        uint32_t wd[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) wd[k] = quant(sv[4 * hh + k]);
-        *(g_u32x4_w*)(row + 16 * hh) = u32x4_t{wd[0], wd[1], wd[2], wd[3]};
+          for (int e = 0; e < 4; ++e) mx = fmaxf(mx, fabsf(q[c][e]));
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        if (mx > 0x1p-80f && mx < 0x1p80f) {
+          int ex;
+          (void)frexpf(mx, &ex);
+          up = ldexpf(1.f, 14 - ex);
+          down = ldexpf(1.f, ex - 14);
+        }
       }
-    };
-    if (quotient_fast(am_bits, s32)) {
-      const double r64 = 1.0 / (double)s32;
-      store_codes([&](const f32x4_t& v) {
-        return f32x4_to_fp8(quotient_f64(v[0], r64), quotient_f64(v[1], r64), quotient_f64(v[2], r64),
-                            quotient_f64(v[3], r64));
-      });
-    } else {
-      store_codes([&](const f32x4_t& v) {
-        return f32x4_to_fp8_ref_cold(v[0] / s32, v[1] / s32, v[2] / s32, v[3] / s32);
-      });
+      // S_n of the tile's 8 column groups: lane (nn, q4) gets
+      // S_n[row][32 q4 + 4 ct + e], code byte 4 ct + e of its 32; U~ of two
+      // chunks at a time in three parts
+      const float ls = lam * up;
+      const int ko = kLdsX + (4 * q4 + (l16 >> 2)) * kXS + 64 * (l16 & 3);
+      f32x4_t sv[8];
+#pragma unroll
+      for (int ct = 0; ct < 8; ++ct) {
+        float f[4];
+        fp8x4_to_f32(cw[ct >> 2][ct & 3], f);
+        sv[ct] = f32x4_t{ls * f[0], ls * f[1], ls * f[2], ls * f[3]};
+      }
+#pragma unroll
+      for (int hh = 0; hh < NF / 2; ++hh) {
+        u32x4_t ub[3];
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+          const f32x4_t x = q[2 * hh + d] * up;
+          const Split3 s01 = split3_act(x[0], x[1]), s23 = split3_act(x[2], x[3]);
+          ub[0][2 * d] = s01.hi, ub[0][2 * d + 1] = s23.hi;
+          ub[1][2 * d] = s01.mid, ub[1][2 * d + 1] = s23.mid;
+          ub[2][2 * d] = s01.lo, ub[2][2 * d + 1] = s23.lo;
+        }
+        u32x4_t k8[8];
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          // (two groups' K^T operands at a time)
+#pragma unroll
+          for (int ct = 4 * g; ct < 4 * g + 4; ++ct) {
+            const uint2 k0 = kt_read(ko + 2 * NT * hh * kXS + 8 * ct);
+            const uint2 k1 = kt_read(ko + (2 * hh + 1) * NT * kXS + 8 * ct);
+            k8[ct] = u32x4_t{k0.x, k0.y, k1.x, k1.y};
+          }
+#pragma unroll
+          for (int d = 2; d >= 0; --d)
+#pragma unroll
+            for (int ct = 4 * g; ct < 4 * g + 4; ++ct) sv[ct] = mfma16(k8[ct], ub[d], sv[ct]);
+          GDNR_COMPILER_FENCE();
+        }
+      }
+      if constexpr (!kBF16) {
+#pragma unroll
+        for (int ct = 0; ct < 8; ++ct) sv[ct] *= down;
+      }
+      // (the next vblock's codes, while this one is requantised)
+      if (p + 1 < p1) load_codes(p + 1);
+      // the reference quantiser (ref:36-37,83-99), as gdnr_decode.hip applies
+      // it; the vblock's amax over the pair's two tiles through LDS (two slots
+      // in turn: one barrier a vblock)
+      float am = 0.f, am1 = 0.f;
+#pragma unroll
+      for (int ct = 0; ct < 8; ++ct) {
+        am = max3_abs(am, sv[ct][0], sv[ct][1]);
+        am1 = max3_abs(am1, sv[ct][2], sv[ct][3]);
+      }
+      const float am_mine = __uint_as_float(wave_max_u32(__float_as_uint(__builtin_elementwise_maximum(am, am1))));
+      float* const rp = red + NW * (p & 1);
+      if (lane == 0) rp[w] = am_mine;
+      lds_barrier();
+      const uint32_t am_bits = (uint32_t)uni((int)max(__float_as_uint(am_mine), __float_as_uint(rp[w ^ 1])));
+      const float amax = __uint_as_float(am_bits);
+      const float s32 = (amax > 0.0f) ? amax / 448.0f : 1.0f;
+      {
+        o = rows_reduce_scatter(o, 0.f, 0.f, 0.f);
+        if (q4 == 0) Act::st(fo_rows, 32 * p + l16, o * a.out_scale);
+      }
+      uint8_t* const row = fc_rows + (uint32_t)(32 * p + l16) * a.ck_v + 32 * q4;
+      auto store_codes = [&](auto quant) {
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+          uint32_t wd[4];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) wd[k] = quant(sv[4 * hh + k]);
+          *(g_u32x4_w*)(row + 16 * hh) = u32x4_t{wd[0], wd[1], wd[2], wd[3]};
+        }
+      };
+      if (quotient_fast(am_bits, s32)) {
+        const double r64 = 1.0 / (double)s32;
+        store_codes([&](const f32x4_t& v) {
+          return f32x4_to_fp8(quotient_f64(v[0], r64), quotient_f64(v[1], r64), quotient_f64(v[2], r64),
+                              quotient_f64(v[3], r64));
+        });
+      } else {
+        store_codes([&](const f32x4_t& v) {
+          return f32x4_to_fp8_ref_cold(v[0] / s32, v[1] / s32, v[2] / s32, v[3] / s32);
+        });
+      }
+      if (lane == 0 && (w & 1) == 0) *(uint16_t*)(fs_rows + p * a.sc_v) = __builtin_bit_cast(uint16_t, (_Float16)s32);
     }
-    if (lane == 0 && (w & 1) == 0) *(uint16_t*)(fs_rows + p * a.sc_v) = __builtin_bit_cast(uint16_t, (_Float16)s32);
-  }
   };
   if (n <= 2 * NT)
     rebuild(std::integral_constant<int, 2>{});
