@@ -269,20 +269,28 @@ PyObject* host_call(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   });
 }
 
-// A buffer of n contiguous items of `size` bytes behind a Python object.
+// A buffer of contiguous items behind a Python object: int64 (T = int64_t) or
+// bytes (T = uint8_t). The format is checked and not only its size: a float64
+// or uint64 array has 8-byte items too.
+template <class T>
 struct Buffer {
   Py_buffer view{};
   bool ok;
-  Buffer(PyObject* o, Py_ssize_t size, bool writable) {
-    ok = PyObject_GetBuffer(o, &view, writable ? PyBUF_CONTIG : PyBUF_CONTIG_RO) == 0;
-    if (ok && view.itemsize != size) {
-      PyErr_Format(PyExc_TypeError, "expected a buffer of %zd-byte items, got %zd", size, view.itemsize);
-      ok = false;
-    }
+  Buffer(PyObject* o, bool writable) {
+    ok = PyObject_GetBuffer(o, &view, PyBUF_ND | PyBUF_FORMAT | (writable ? PyBUF_WRITABLE : 0)) == 0;
+    if (!ok) return;
+    const char* f = view.format ? view.format : "B";
+    if (*f == '@' || *f == '=') ++f;
+    const bool fits = sizeof(T) == 8 ? (*f == 'l' || *f == 'q') && !f[1] : (*f == 'B' || *f == '?') && !f[1];
+    if (fits && view.itemsize == (Py_ssize_t)sizeof(T)) return;
+    PyErr_Format(PyExc_TypeError, "expected a buffer of %s, got %zd-byte items of format '%s'",
+                 sizeof(T) == 8 ? "8-byte signed integers" : "bytes", view.itemsize, view.format ? view.format : "B");
+    ok = false;
   }
   ~Buffer() {
     if (view.obj) PyBuffer_Release(&view);
   }
+  T* data() const { return (T*)view.buf; }
   Py_ssize_t count() const { return view.len / view.itemsize; }
 };
 
@@ -297,20 +305,20 @@ PyObject* host_slot_metadata(PyObject*, PyObject* const* args, Py_ssize_t nargs)
   }
   const long long window = PyLong_AsLongLong(args[2]);
   if (window == -1 && PyErr_Occurred()) return nullptr;
-  Buffer fill(args[0], 8, false);
+  const Buffer<int64_t> fill(args[0], false);
   if (!fill.ok) return nullptr;
-  Buffer slots(args[1], 8, false);
+  const Buffer<int64_t> slots(args[1], false);
   if (!slots.ok) return nullptr;
-  Buffer out(args[3], 1, true);
+  const Buffer<uint8_t> out(args[3], true);
   if (!out.ok) return nullptr;
   return guarded([&]() -> PyObject* {
     const Py_ssize_t n = slots.count(), total = fill.count();
-    const int64_t *f = (const int64_t*)fill.view.buf, *s = (const int64_t*)slots.view.buf;
+    const int64_t *f = fill.data(), *s = slots.data();
     if (out.count() < 13 * n) {
       PyErr_SetString(PyExc_ValueError, "out is too small");
       return nullptr;
     }
-    int32_t* o = (int32_t*)out.view.buf;
+    int32_t* o = (int32_t*)out.data();
     uint8_t* flush = (uint8_t*)(o + 3 * n);
     std::vector<bool> seen(total);
     for (Py_ssize_t i = 0; i < n; ++i)
@@ -342,12 +350,12 @@ PyObject* host_advance(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   }
   const long long window = PyLong_AsLongLong(args[2]);
   if (window == -1 && PyErr_Occurred()) return nullptr;
-  Buffer fill(args[0], 8, true);
+  const Buffer<int64_t> fill(args[0], true);
   if (!fill.ok) return nullptr;
-  Buffer slots(args[1], 8, false);
+  const Buffer<int64_t> slots(args[1], false);
   if (!slots.ok) return nullptr;
-  int64_t* f = (int64_t*)fill.view.buf;
-  const int64_t* s = (const int64_t*)slots.view.buf;
+  int64_t* f = fill.data();
+  const int64_t* s = slots.data();
   const Py_ssize_t total = fill.count();
   for (Py_ssize_t i = 0; i < slots.count(); ++i)
     if (s[i] > 0 && s[i] < total) f[s[i]] = f[s[i]] + 1 == window ? 0 : f[s[i]] + 1;

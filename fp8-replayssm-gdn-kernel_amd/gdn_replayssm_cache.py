@@ -107,11 +107,14 @@ class ReplaySSMCache:
         if slots.ndim != 1:
             raise ValueError("slots must be one-dimensional")
         host = gdnr_lib.host()
+        # (the extension takes int64 fills; an array of another type that
+        # replaced them steps on a copy)
+        fill = np.ascontiguousarray(self.fill, dtype=np.int64)
         batch = slots.shape[0]
         # slot, pos, valid_len (int32) and flush (a byte) of each entry, in one
         # pinned buffer and one copy
         packed = torch.empty(13 * batch, dtype=torch.uint8, pin_memory=True)
-        host.slot_metadata(self.fill, slots, self.window, packed.numpy())
+        host.slot_metadata(fill, slots, self.window, packed.numpy())
         if mixed_qkv.shape[0] != batch:
             raise ValueError(f"mixed_qkv has {mixed_qkv.shape[0]} rows for a batch of {batch}")
         packed = packed.to(self.device, non_blocking=True)
@@ -121,5 +124,7 @@ class ReplaySSMCache:
         result = gk.gdn_prep_replay_fp8(mixed_qkv, a, b, a_log, dt_bias, meta[1], self.payload, self.scale, q_out,
                                         self.k_ring, self.v_ring, self.g_ring, self.beta_ring, meta[2],
                                         packed[12 * batch:], block_v=block_v, out=out, state_indices=meta[0])
-        host.advance(self.fill, slots, self.window)
+        host.advance(fill, slots, self.window)
+        if fill is not self.fill:
+            self.fill[slots] = fill[slots]
         return result

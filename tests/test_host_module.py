@@ -70,3 +70,52 @@ def test_call_errors(host):
     assert error.value.status == 1
     with pytest.raises(TypeError, match="3 tensors"):
         gdnr_lib.call("gdnr_dequantize_vblock32", [codes, scale])
+
+
+class _Launch:
+    """step()'s launch replaced by a note of the metadata it was given (with
+    pageable buffers: there is no GPU to pin for)."""
+
+    def __init__(self, monkeypatch):
+        empty = torch.empty
+        monkeypatch.setattr(torch, "empty", lambda *shape, pin_memory=False, **kw: empty(*shape, **kw))
+        monkeypatch.setattr(gk, "gdn_prep_replay_fp8", self)
+
+    def __call__(self, mixed, a, b, a_log, dt_bias, pos, *rest, state_indices, **kw):
+        self.slots, self.pos, self.valid, self.flush = state_indices, pos, rest[7], rest[8]
+        return mixed
+
+
+def _cpu_cache(window=4):
+    return ReplaySSMCache(5, window, heads=1, value_heads=1, key_dim=128, value_dim=32, device="cpu")
+
+
+def _cpu_step(cache, slots):
+    rows = torch.zeros(len(slots), 1)
+    return cache.step(slots, rows, rows, rows, rows[:0], rows[:0])
+
+
+def test_buffers_of_other_formats_are_refused(host):
+    slots, packed = np.array([1], np.int64), np.zeros(64, np.uint8)
+    for fill in (np.full(4, 2.0), np.full(4, 2, np.uint64), np.zeros(4, ">i8")):
+        with pytest.raises(TypeError, match="8-byte signed"):
+            host.slot_metadata(fill, slots, 4, packed)
+        with pytest.raises(TypeError, match="8-byte signed"):
+            host.advance(fill, slots, 4)
+    with pytest.raises(TypeError, match="bytes"):
+        host.slot_metadata(np.zeros(4, np.int64), slots, 4, np.zeros(16, np.int32))
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64, np.uint64, np.float64])
+def test_step_takes_fills_of_any_dtype(host, monkeypatch, dtype):
+    """A cache whose fill array was replaced (restored from a file, say) steps
+    as metadata() says, whatever its dtype."""
+    launch, cache = _Launch(monkeypatch), _cpu_cache()
+    cache.fill = np.array([0, 2, 0, 3, 0, 0], dtype)
+    for pos, flush in (([2, -1, 3], [0, 0, 1]), ([3, -1, 0], [1, 0, 0]), ([0, -1, 1], [0, 0, 0])):
+        want = cache.metadata([1, 0, 3])
+        _cpu_step(cache, [1, 0, 3])
+        got = (launch.slots, launch.pos, launch.valid, launch.flush)
+        assert launch.pos.tolist() == pos and launch.flush.tolist() == flush
+        assert all(np.array_equal(np.asarray(x), y.astype(np.int32)) for x, y in zip(got, want))
+    assert cache.fill.dtype == dtype and cache.fill.tolist() == [0, 1, 0, 2, 0, 0]
