@@ -103,9 +103,10 @@ class ReplaySSMCache:
         """One full-contract decode step of the batch: batch entry i is the
         sequence in slot slots[i] (0 = padding; its output is meaningless).
         mixed_qkv [B, 2HK + HV V], a, b [B, HV]; returns out [B, HV, V]."""
-        slots = np.ascontiguousarray(slots, dtype=np.int64)
-        if slots.ndim != 1:
+        slots = np.asarray(slots, dtype=np.int64)
+        if slots.ndim != 1:  # (ascontiguousarray makes a scalar a vector)
             raise ValueError("slots must be one-dimensional")
+        slots = np.ascontiguousarray(slots)
         host = gdnr_lib.host()
         # (the extension takes int64 fills; an array of another type that
         # replaced them steps on a copy)

@@ -119,3 +119,10 @@ def test_step_takes_fills_of_any_dtype(host, monkeypatch, dtype):
         assert launch.pos.tolist() == pos and launch.flush.tolist() == flush
         assert all(np.array_equal(np.asarray(x), y.astype(np.int32)) for x, y in zip(got, want))
     assert cache.fill.dtype == dtype and cache.fill.tolist() == [0, 1, 0, 2, 0, 0]
+
+
+@pytest.mark.parametrize("slots", [5, np.int64(5), np.array(5), [[1, 2]]])
+def test_step_refuses_slots_that_are_no_vector(host, monkeypatch, slots):
+    _Launch(monkeypatch)
+    with pytest.raises(ValueError, match="one-dimensional"):
+        _cpu_cache().step(slots, *[torch.zeros(1, 1)] * 5)
