@@ -114,7 +114,7 @@ class ReplaySSMCache:
         batch = slots.shape[0]
         # slot, pos, valid_len (int32) and flush (a byte) of each entry, in one
         # pinned buffer and one copy
-        packed = torch.empty(13 * batch, dtype=torch.uint8, pin_memory=True)
+        packed = torch.empty(13 * batch, dtype=torch.uint8, device="cpu", pin_memory=True)
         host.slot_metadata(fill, slots, self.window, packed.numpy())
         if mixed_qkv.shape[0] != batch:
             raise ValueError(f"mixed_qkv has {mixed_qkv.shape[0]} rows for a batch of {batch}")

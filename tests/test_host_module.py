@@ -78,6 +78,8 @@ class _Launch:
 
     def __init__(self, monkeypatch):
         empty = torch.empty
+        with torch.device("cpu"):  # (torch lists its factories at the first use of a default device)
+            empty(0)
         monkeypatch.setattr(torch, "empty", lambda *shape, pin_memory=False, **kw: empty(*shape, **kw))
         monkeypatch.setattr(gk, "gdn_prep_replay_fp8", self)
 
@@ -126,3 +128,13 @@ def test_step_refuses_slots_that_are_no_vector(host, monkeypatch, slots):
     _Launch(monkeypatch)
     with pytest.raises(ValueError, match="one-dimensional"):
         _cpu_cache().step(slots, *[torch.zeros(1, 1)] * 5)
+
+
+def test_step_packs_on_the_host_under_any_default_device(host, monkeypatch):
+    """torch.empty follows torch's default device; the packed metadata is host
+    memory under any."""
+    launch, cache = _Launch(monkeypatch), _cpu_cache()
+    rows = torch.zeros(2, 1)
+    with torch.device("meta"):
+        cache.step([3, 0], rows, rows, rows, rows[:0], rows[:0], q_out=rows)
+    assert launch.pos.tolist() == [0, -1] and launch.valid.tolist() == [1, 0]
