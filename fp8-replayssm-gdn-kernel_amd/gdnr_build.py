@@ -28,8 +28,15 @@ LIBRARY = PKG_DIR / "libgdnreplay.so"
 HOST_MODULE = PKG_DIR / "_gdnr_host.so"
 ARCH = os.environ.get("GDNR_OFFLOAD_ARCH", "gfx950")
 
-ROCM = Path("/opt/rocm")
-HIPCC = shutil.which("hipcc") or str(ROCM / "bin/hipcc")
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+
+
+def _rocm() -> Path:
+    """The ROCm tree hipcc belongs to (its headers go with its compiler)."""
+    tree = Path(HIPCC).resolve().parents[1]
+    return tree if (tree / "include/hip/hip_runtime_api.h").exists() else Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
+
+
 DEVICE_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -67,7 +74,7 @@ def _host_module_job(out: Path) -> list[str]:
     return ["g++", *HOST_FLAGS, "-Wno-unused-parameter", "-shared", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__=1",
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{INCLUDE}",
             f"-I{sysconfig.get_paths()['include']}", f"-isystem{root / 'include'}",
-            f"-isystem{root / 'include/torch/csrc/api/include'}", f"-isystem{ROCM / 'include'}",
+            f"-isystem{root / 'include/torch/csrc/api/include'}", f"-isystem{_rocm() / 'include'}",
             str(CSRC / "gdnr_host.cpp"), "-o", str(out), f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10",
             "-lc10_hip"]
 
@@ -89,15 +96,23 @@ def build(verbose: bool = False) -> Path:
     abi_obj = BUILD_DIR / "gdnr_abi.o"
     jobs.append(["g++", *HOST_FLAGS, *inc, "-c", str(CSRC / "gdnr_abi.cpp"), "-o", str(abi_obj)])
     host_tmp = HOST_MODULE.with_name(HOST_MODULE.name + ".tmp")
-    jobs.append(_host_module_job(host_tmp))
-    with ThreadPoolExecutor(max_workers=len(jobs)) as pool:
+    with ThreadPoolExecutor(max_workers=len(jobs) + 1) as pool:
+        # the library needs neither torch nor the module: a host without torch's
+        # or Python's headers still gets it
+        try:
+            host_module = pool.submit(_run, _host_module_job(host_tmp), verbose)
+        except ImportError:
+            host_module = None
+            print(f"torch is not importable: {HOST_MODULE.name} is not built", file=sys.stderr)
         for future in [pool.submit(_run, cmd, verbose) for cmd in jobs]:
             future.result()
     tmp = LIBRARY.with_name(LIBRARY.name + ".tmp")
     _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, kern_objs), str(abi_obj), "-o", str(tmp)],
          verbose)
     tmp.replace(LIBRARY)
-    host_tmp.replace(HOST_MODULE)
+    if host_module:
+        host_module.result()
+        host_tmp.replace(HOST_MODULE)
     return LIBRARY
 
 
