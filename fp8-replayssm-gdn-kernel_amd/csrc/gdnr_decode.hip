@@ -43,6 +43,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #ifndef GDNR_ACT
@@ -238,7 +239,7 @@ __global__ __launch_bounds__(768) __attribute__((amdgpu_waves_per_eu(3))) void d
   const int w = uni(threadIdx.x >> 6);
   const int gw = shape & 0xFF, U = (shape >> 8) & 0xFF;  // value heads per unit, units per workgroup
   // workgroups numbered sequence-fastest (grid x = sequences) or head-fastest
-  const bool seq_major = (shape >> 16) != 0;
+  const bool seq_major = ((shape >> 16) & 1) != 0;
   const int bx = (int)(seq_major ? blockIdx.y : blockIdx.x), by = (int)(seq_major ? blockIdx.x : blockIdx.y);
   const int rpu = gw * NWH;                     // row waves per unit
   const bool chain = w < U;                     // waves [0, U): the chain waves
@@ -254,22 +255,29 @@ __global__ __launch_bounds__(768) __attribute__((amdgpu_waves_per_eu(3))) void d
   const int n_grp = uni(G / gw);
   const int h = uni(r / n_grp), grp = r - h * n_grp;
   int b0 = uni(by * SP + us);
-  // SWAP (launches of many rounds of workgroups, one unit each): sequences b
-  // and B - 1 - b change places when only the later one flushes. A flush runs
-  // several times as long as a replay; one that starts in the launch's last
-  // rounds ends it late (B=512, L=8, 64 flushes spread over the batch 79.3 us,
-  // so 70.2; B=256, L=16, 16 of them 41.4 and 36.5; no flush at all 61.6 and
-  // 62.2). An instantiation of its own: the flags' loads in the others' prologue
-  // cost them 1 to 3%.
+  // SWAP (launches of many rounds of workgroups, one unit each): past the
+  // first round's sequences [0, first), sequences b and first + B - 1 - b
+  // change places when only the later one flushes. A flush runs several times
+  // as long as a replay; one that starts in the launch's last rounds ends it
+  // late (us a launch in the batch's order and swapped, fills spread over the
+  // batch: B=256, L=16 39.5 and 36.9; B=512, L=8 74.3 and 72.4). The flags'
+  // loads come before a wave's first request, which other workgroups' streams
+  // hide, but not in the first round (launches without a flush, in the batch's
+  // order, with every sequence swapped, and without the first round's: B=256,
+  // L=16 34.6, 35.6 and 34.8; B=512, L=8 63.0, 63.6 and 63.3; a lockstep cycle
+  // of B=256, L=16 37.9, 38.5 and 37.8).
   if constexpr (SWAP) {
-    const int other = a.B - 1 - b0;
-    auto flushes = [&](int bq) {
-      const uintptr_t fa = (uintptr_t)(a.flush + (uint32_t)bq * a.fl_s);
-      const uint32_t word = ld_u32_uniform((const void*)(fa & ~(uintptr_t)3));
-      return uni((int)((word >> (8u * (uint32_t)(fa & 3))) & 0xFFu)) != 0;
-    };
-    const bool late = flushes(max(b0, other)), early = flushes(min(b0, other));
-    b0 = late && !early ? other : b0;
+    const int first = shape >> 17;
+    if (b0 >= first) {
+      const int other = first + a.B - 1 - b0;
+      auto flushes = [&](int bq) {
+        const uintptr_t fa = (uintptr_t)(a.flush + (uint32_t)bq * a.fl_s);
+        const uint32_t word = ld_u32_uniform((const void*)(fa & ~(uintptr_t)3));
+        return uni((int)((word >> (8u * (uint32_t)(fa & 3))) & 0xFFu)) != 0;
+      };
+      const bool late = flushes(max(b0, other)), early = flushes(min(b0, other));
+      b0 = late && !early ? other : b0;
+    }
   }
   const int hv0 = h * G + grp * gw;              // first value head of the unit
   uint8_t* const ul = lds + u * unit_lds(NCH, rpu, TPW / 2);  // the unit's LDS block
@@ -1615,13 +1623,16 @@ int launch_variant(const StepArgs& a, hipStream_t s) {
   const dim3 grid(seq_major ? gs : gh, seq_major ? gh : gs),
       block((unsigned)(64 * a.units * (1 + a.gw * NWH)));
   auto kernel = decode_kernel<TPW, NWH, NCH, FUSED, GATE_F32, SLOTS, SWAP>;
+  // the sequences of a swapping launch's first round of workgroups (12 waves
+  // per compute unit)
+  const unsigned first = SWAP ? std::min(12u / (1 + a.gw * NWH) * (unsigned)device_cus() / gh, 0x3FFFu) : 0;
   if (a.lds_bytes > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, a.lds_bytes);
     if (e != hipSuccess) return (int)e;
   }
   hipLaunchKernelGGL(kernel, grid, block, a.lds_bytes, s, a.ckpt, a.k, a.ck_b, a.ck_h, a.ck_v, a.k_b, a.k_t, a.k_h,
-                     a.L, a.G, a.gw | (a.units << 8) | ((seq_major ? 1 : 0) << 16), a);
+                     a.L, a.G, a.gw | (a.units << 8) | ((seq_major ? 1 : 0) << 16) | (int)(first << 17), a);
   return 0;
 }
 
