@@ -268,3 +268,69 @@ def test_decode_flush_requantiser_bit_exact(device, case, fused):
         total += gs.size
     # the quotients were real divisions: most scales changed
     assert changed > 0.9 * total, (changed, total)
+
+
+# ---------------------------------------------------------------------------
+# ... and on the ring kernel (csrc/gdnr_ring.hip: 16-bit rings of 17 to 64
+# tokens past the decode kernel's batches): each of its workgroup shapes, two
+# and four chunks, whole flushes and (a few flushing sequences in a launch of
+# more than one round) flushes in halves.
+# ---------------------------------------------------------------------------
+
+RING_CASES = {
+    # id: (batch, heads, value_heads, value_dim, ring, dtype, flush pattern)
+    "two_waves_all": (64, 16, 32, 128, 64, torch.bfloat16, "all"),
+    "two_waves_two_chunks": (64, 16, 32, 128, 32, torch.float16, "alternate"),
+    "two_waves_halves": (64, 16, 32, 128, 64, torch.bfloat16, "few"),
+    "two_waves_halves_f16": (50, 16, 32, 128, 48, torch.float16, "few"),
+    "four_waves_one_round": (20, 16, 32, 128, 64, torch.bfloat16, "all"),
+    "four_waves_halves": (40, 16, 32, 128, 40, torch.float16, "few"),
+    "V64": (80, 16, 32, 64, 48, torch.bfloat16, "few"),
+    "V256": (20, 8, 8, 256, 40, torch.bfloat16, "alternate"),
+    "odd_group": (44, 4, 12, 128, 17, torch.float16, "alternate"),
+}
+
+
+@pytest.mark.parametrize("fused", [False, True], ids=["replay", "prep_replay"])
+@pytest.mark.parametrize("case", list(RING_CASES))
+def test_ring_flush_requantiser_bit_exact(device, case, fused):
+    import gdnr_lib
+
+    batch, heads, value_heads, value_dim, ring, act, pattern = RING_CASES[case]
+    assert gdnr_lib.decode_plan(batch, heads, value_heads, value_dim, ring, act=act) is None
+    codes0, scale0, nan_blocks = _device_checkpoint(batch, value_heads, value_dim, seed=batch + ring, device=device)
+    flush = torch.zeros(batch, dtype=torch.bool, device=device)
+    flush[[0, 2, 7, 31, batch - 2, batch - 1] if batch > 31 else [0, 2, 7, batch - 2, batch - 1]] = True
+    if pattern != "few":
+        flush[::1 if pattern == "all" else 2] = True
+    assert all(flush[b] for b, _, _ in nan_blocks)
+    gen = torch.Generator(device=device).manual_seed(12)
+    rings = [torch.randn(batch, ring, heads, K, generator=gen, device=device).to(act),
+             torch.randn(batch, ring, value_heads, value_dim, generator=gen, device=device).to(act),
+             torch.zeros(batch, ring, value_heads, dtype=act, device=device),
+             torch.zeros(batch, ring, value_heads, dtype=act, device=device)]
+    # full rings mostly, every third sequence at some other fill
+    valid = torch.randint(1, ring + 1, (batch,), generator=gen, device=device)
+    valid = torch.where(torch.arange(batch, device=device) % 3 == 2, valid, ring).to(torch.int32)
+    payload, scale = codes0.clone().view(torch.float8_e4m3fn), scale0.clone()
+    if fused:
+        mixed = torch.randn(batch, 2 * heads * K + value_heads * value_dim, generator=gen, device=device).to(act)
+        a = torch.randn(batch, value_heads, generator=gen, device=device).to(act)
+        b = torch.full((batch, value_heads), -float("inf"), dtype=act, device=device)
+        a_log = torch.full((value_heads,), -float("inf"), device=device)
+        q_out = torch.empty(batch, heads, K, dtype=act, device=device)
+        gk.gdn_prep_replay_fp8(mixed, a, b, a_log, torch.zeros(value_heads, device=device), valid - 1, payload, scale,
+                               q_out, *rings, valid, flush, block_v=min(128, value_dim))
+    else:
+        q = torch.randn(batch, heads, K, generator=gen, device=device).to(act)
+        gk.gdn_replay_fp8(payload, scale, q, *rings, valid, flush, block_v=32)
+    got = payload.view(torch.uint8)
+    assert torch.equal(got[~flush], codes0[~flush]) and torch.equal(scale[~flush], scale0[~flush])
+    seqs = np.nonzero(flush.cpu().numpy())[0]
+    want_codes, want_scale = _expected_requant(codes0, scale0, seqs)
+    bad = _zero_sign_free(got[flush].cpu().numpy()) != _zero_sign_free(want_codes)
+    assert not bad.any(), (case, int(bad.sum()), np.argwhere(bad)[:4])
+    got_scale = scale[flush].cpu().numpy()
+    assert np.array_equal(got_scale.view(np.uint16), want_scale.view(np.uint16)), case
+    # the quotients were real divisions: most scales changed
+    assert np.mean(got_scale != scale0[flush].cpu().numpy()) > 0.9

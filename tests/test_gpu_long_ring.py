@@ -1,8 +1,8 @@
 """GPU parity of the long-ring full-contract path (marked `gpu`): rings of 17
 to 64 tokens, which gdn_prep_replay_fp8 runs on the decode kernel's chunked
 path at small batches (csrc/gdnr_decode.hip, up to 16 sequences of 32 value
-heads) and on the fused replay kernel beyond (prep + replay or flush in one
-launch, csrc/gdnr_kernels.hip).
+heads), on the ring kernel beyond (csrc/gdnr_ring.hip), and on the fused
+replay kernel (csrc/gdnr_kernels.hip) for the shapes that neither holds.
 
 The reference's full-contract cycle (prototype/bench_gdn_full_contract.py
 :225-308) over a little more than one ring with mixed ring phases, so that
@@ -47,7 +47,7 @@ def _within_bf16_ulp(got, want):
     return bool(np.all(np.abs(got - want) <= ulp)) and float(np.mean(got != want)) < 0.01
 
 
-@pytest.mark.parametrize("batch", [3, 20], ids=["decode_kernel", "replay_kernel"])
+@pytest.mark.parametrize("batch", [3, 20], ids=["decode_kernel", "ring_kernel"])
 @pytest.mark.parametrize("window", [32, 64])
 def test_long_ring_cycle_matches_oracle(device, window, batch):
     import gdnr_lib
@@ -141,3 +141,65 @@ def test_long_ring_tiles_identical(device):
     for other in results[1:]:
         for x, y in zip(results[0], other):
             assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("batch,heads,value_heads,value_dim,window", [
+    (9, 4, 8, 96, 33), (9, 4, 8, 32, 64), (43, 4, 12, 64, 64), (43, 4, 12, 64, 17)])
+def test_replay_kernel_16_bit(device, batch, heads, value_heads, value_dim, window, dtype):
+    """The shapes of 16-bit rings that neither the decode kernel nor the ring
+    kernel holds (V = 32, 96, ...; V = 64 with an odd group past the decode
+    kernel's batches): replays and flushes at fills around the 16-token
+    chunks against the fp64 oracle; the fused launch and the slot-indexed one
+    against prep then replay, bit for bit. Outputs 2e-3 rel-L2 over the batch;
+    a single sequence's few hundred values, in which a few large ones can
+    weigh most, within bf16's largest rounding, 2^-8 of each value."""
+    from gpu_helpers import make_replay_case, oracle_replay, run_replay
+    import gdnr_lib
+
+    assert gdnr_lib.decode_plan(batch, heads, value_heads, value_dim, window, act=dtype) is None
+    assert value_dim not in (64, 128, 256) or (value_dim == 64 and value_heads // heads % 2)  # (not the ring kernel's)
+    edges = [window, 1, 16, 17, window - 1, 0]
+    valid = np.array([edges[i % len(edges)] for i in range(batch)])
+    flush = np.array([i % 2 == 0 for i in range(batch)])
+    block_v = 64 if value_dim % 64 == 0 else 32
+    case = make_replay_case(batch, window, device, seed=4400, heads=heads, value_heads=value_heads, value_dim=value_dim,
+                            dtype=dtype, warmup=8, valid=valid, flush=flush, reference_dist=True)
+    shape = synth.Shape(batch, heads, value_heads, value_dim=value_dim)
+    gen = synth.generator(4401, device)
+    a_log, dt_bias = synth.gating_params(shape, gen, device, reference_dist=True)
+    mixed, a, b = (t[:, 0].contiguous() for t in synth.raw_step_inputs(shape, 1, gen, device, dtype, dtype))
+    pos = torch.as_tensor(np.maximum(valid - 1, 0), dtype=torch.int32, device=device)
+    slots = torch.randperm(batch, generator=torch.Generator().manual_seed(4)).to(device) + 1
+    results = []
+    for mode in ("pair", "fused", "slots"):
+        state = [case["ckpt"].payload.view(torch.uint8).clone(), case["ckpt"].scale.clone(),
+                 *(case[k].clone() for k in ("k", "v", "g", "beta"))]
+        if mode == "slots":
+            cache = [torch.zeros(batch + 1, *t.shape[1:], dtype=t.dtype, device=device) for t in state]
+            for c, t in zip(cache, state):
+                c[slots] = t
+            state = cache
+        payload, scale, *rings = state
+        payload, q_out = payload.view(torch.float8_e4m3fn), torch.zeros_like(case["q"])
+        if mode == "pair":
+            gk.gdn_prep_ring(mixed, a, b, a_log, dt_bias, pos, q_out, *rings)
+            out = gk.gdn_replay_fp8(payload, scale, q_out, *rings, case["valid"], case["flush"], block_v=block_v)
+        else:
+            out = gk.gdn_prep_replay_fp8(mixed, a, b, a_log, dt_bias, pos, payload, scale, q_out, *rings, case["valid"],
+                                         case["flush"], block_v=block_v,
+                                         state_indices=slots if mode == "slots" else None)
+        results.append([out, q_out, *(t[slots] if mode == "slots" else t for t in (payload.view(torch.uint8), scale, *rings))])
+    for other in results[1:]:
+        for x, y in zip(results[0], other):
+            assert torch.equal(x, y)
+
+    out = np32(run_replay(case, block_v=block_v))
+    ref, ref_codes, ref_scale = oracle_replay(case)
+    codes, scale = codes_np(case["ckpt"].payload), case["ckpt"].scale.cpu().numpy()
+    assert np.array_equal(codes[~flush], case["codes0"][~flush]) and np.array_equal(scale[~flush], case["scale0"][~flush])
+    assert rel_l2(out, ref) <= OUT_TOL
+    for i in range(batch):
+        assert rel_l2(out[i], ref[i]) <= 2.0 ** -8, (i, valid[i], flush[i])
+    assert np.mean(codes != ref_codes) < 1e-4
+    assert np.abs(scale.view(np.int16).astype(np.int32) - ref_scale.view(np.int16).astype(np.int32)).max() <= 1

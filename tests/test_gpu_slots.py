@@ -27,7 +27,7 @@ from oracle import gdn_oracle
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("L,nseq", [(8, 8), (32, 8), (64, 8), (64, 17)])
+@pytest.mark.parametrize("L,nseq", [(8, 8), (32, 8), (64, 8), (64, 17), (48, 40), (33, 60), (8, 258)])
 def test_slots_equal_direct_path(device, L, nseq):
     """nseq sequences live in scattered slots of a cache of nseq + 4 slots
     (8: slots 9, 2, 5, 11, 1, 7, 4, 10 of 12); the batch also carries two
@@ -35,8 +35,10 @@ def test_slots_equal_direct_path(device, L, nseq):
     sequence flushes twice): every output, ring row and checkpoint byte
     equals the direct path's on batch-ordered copies. L = 8 runs the decode
     kernel, L = 32 and 64 with 8 sequences its chunked path (10 batch entries
-    of 32 value heads); 17 sequences at L = 64 the long-ring kernel (slots and
-    direct path both past the decode kernel's 16 sequences)."""
+    of 32 value heads); 17 and more sequences at L > 16 the ring kernel (17 in
+    one round of workgroups; 40 and 60 in several, flushing sequences first,
+    four and two waves a head); 258 at L = 8 the decode kernel's plan for large
+    launches, late flushes swapped forward."""
     B, steps = nseq, (5 * L) // 2
     shape = synth.Shape(B)
     gen = synth.generator(61, device)
