@@ -26,11 +26,18 @@
 // row sums reduce across the row's lanes with DPP (plus one swizzle for
 // 32-lane rows). Loads and stores are non-temporal: a layer's state is next
 // touched a whole step later, after every other layer's. Measured on MI355X
-// (us a step of a bf16 state, HV=32, V=128, rotating states past the Infinity
-// Cache; before: plain accesses, 32 rows a wave): B=64 25.1 (33.0), B=32 12.5
-// (18.6), B=8 5.5 (8.2), B=1 3.8 (5.3); f32 B=64 49.4 (61.2), B=16 12.0 (17.7).
-// 5.3 TB/s read + written at B=64. A state that stays in that cache from step
-// to step (one layer alone) gains nothing or loses some: B=64 22.9 (22.6).
+// (us a step of a bf16 state, HV=32, V=128; before: plain accesses, 32 rows a
+// wave), 12 layers' states in turn, past the 256 MB Infinity Cache from B=21:
+// B=8 5.5 (7.5), B=24 10.0 (15.2), B=32 12.0 (18.9), B=48 20.4 (24.8), B=64
+// 26.1 (33.3; 5.1 TB/s read + written), B=96 40.5 (47.6), B=128 52.2 (61.3);
+// f32 B=16 12.3 (18.2), B=32 26.7 (31.6), B=64 49.7 (61.5).
+// The price: states of a few layers that fit that cache together are no longer
+// served from it, and from 25 MB a layer on the cache is faster than HBM: one
+// layer of B=32 13.9 (12.5), B=64 24.4 (24.2), B=96 40.4 (33.7), f32 B=64 51.2
+// (42.9); three of B=48 20.7 (18.7), B=64 27.0 (24.2). A launch cannot tell how
+// many layers its caller steps; models have them by the dozen. (Plain loads or
+// plain stores alone, and a part of every state plain, lose as much there or
+// gain nothing past the cache: B=64 with plain stores 25 to 26 and 31.3.)
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -194,15 +201,21 @@ void launch_height(const RmwArgs& a, hipStream_t s) {
 }
 
 // Rows per wave (a divisor of V: a wave's rows stay in one head): 4 KiB of a
-// row block, so that a small batch covers the chip; 16 KiB of a 2-byte state
-// once that leaves at least three workgroups per compute unit (us at 64 and 16
-// rows: B=32 15.0 and 12.5, B=48 19.8 and 20.6, B=64 25.1 and 27.3, B=128 53.0
-// and 51.9 to 54.3; an f32 state at 32 and 8 rows: B=64 51.7 and 49.4).
+// row block, so that a small batch covers the chip. 16 KiB of a 2-byte state
+// where those workgroups are resident at once, and nearly as many on every
+// compute unit (three or four; the registers of 64 rows leave room for four):
+// a launch takes as long as its fullest unit. us at 16 and 64 rows, 12 layers
+// in turn: B=32 (two a unit) 11.9 and 15.1, B=44 20.5 and 20.0, B=48 (three)
+// 21.5 and 20.4, B=56 24.4 and 25.9, B=60 26.7 and 25.7, B=64 (four) 28.0 and
+// 26.3, B=68 29.5 and 31.9, B=96 40.6 and 44.0, B=128 52.3 and 54.0. An f32
+// state at 8 and 32 rows: B=16 12.3 and 14.3, B=64 49.8 and 52.6 (B=24 to 32
+// the other way: 26.7 and 25.1).
 template <class S, class Act, bool PACKED = false, bool GATE_F32 = false>
 void launch_rows(const RmwArgs& a, hipStream_t s) {
+  const int64_t tall = ((int64_t)a.B * a.HV * a.V + 255) / 256, cus = device_cus(), per_cu = (tall + cus - 1) / cus;
   if constexpr (S::kBytes == 4) {
     launch_height<S, Act, 8, PACKED, GATE_F32>(a, s);
-  } else if (a.V % 64 == 0 && (int64_t)a.B * a.HV * a.V >= 3 * 256 * (int64_t)device_cus()) {
+  } else if (a.V % 64 == 0 && (per_cu == 3 || per_cu == 4) && 16 * tall >= 15 * per_cu * cus) {
     launch_height<S, Act, 64, PACKED, GATE_F32>(a, s);
   } else {
     launch_height<S, Act, 16, PACKED, GATE_F32>(a, s);

@@ -17,7 +17,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("batch,heads,value_heads,value_dim,state", [
-    (48, 16, 32, 128, torch.bfloat16), (47, 16, 32, 128, torch.bfloat16), (130, 8, 16, 96, torch.float16),
+    (48, 16, 32, 128, torch.bfloat16), (47, 16, 32, 128, torch.bfloat16), (60, 16, 32, 128, torch.bfloat16),
+    (65, 16, 32, 128, torch.float16), (130, 8, 16, 96, torch.float16),
     (128, 4, 12, 128, torch.float16), (5, 1, 3, 32, torch.bfloat16), (48, 16, 32, 128, torch.float32),
     (3, 2, 2, 96, torch.float32)])
 def test_row_blocks(device, batch, heads, value_heads, value_dim, state):
