@@ -255,18 +255,13 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
     if (bs < 0 || bs >= a.n_slots) bs = 0;
 
   // ---- requests: the wave's 16 key rows in the X operand layout, the query
-  // (and new key) row, the gates by token, then the codes (and a replay's v
-  // rows). Nothing past the fill's end is asked for: requests of token 0 in
-  // its place, from the cache, cost a short fill 2 to 4% (B=200, L=17 at fill 8
-  // 38.0 us, so 36.7; V=256, one sequence of 8 heads at fill 1 5.7 and 5.5).
+  // (and new key) row, the gates by token, then the codes
   const int tw = NT * w + l16;            // the key row this lane stages
   u32x4_t kx[4];
   {
     const uint8_t* krow = sbase(a.k, bs, a.k_b) + (h * a.k_h + (uint32_t)(tw < n ? tw : 0) * a.k_t) + 64 * q4;
-    if (NT * w < n) {
 #pragma unroll
-      for (int m = 0; m < 4; ++m) kx[m] = ld16(krow + 16 * m);
-    }
+    for (int m = 0; m < 4; ++m) kx[m] = ld16(krow + 16 * m);
   }
   uint32_t qbits, kbits = 0, ab0 = 0, ab1 = 0;
   float alog = 0.f, dtb = 0.f;
@@ -400,7 +395,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
     const int vp = lane % CPT, vt = lane / CPT;
 #pragma unroll
     for (int k = 0; k < NVL; ++k) {
-      if (k * TPL >= n) break;
       const int t = k * TPL + vt;
       vq[k] = *(g_u32x4*)(v_rows + ((uint32_t)(t < n ? t : 0) * a.v_t + 16 * vp));
     }
