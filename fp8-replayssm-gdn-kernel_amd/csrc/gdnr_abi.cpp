@@ -480,8 +480,12 @@ void fill_index(const gdnr_tensor* t, const T** p, int64_t* s) {
 bool decode_eligible(const gdnr::ReplayArgs& a, int act) {
   if (act != GDNR_DTYPE_BF16 && act != GDNR_DTYPE_F16) return false;
   if (a.L <= gdnr::kStepRing) return a.V == 64 || a.V == 128 || a.V == 256;
-  // (a ring of chunks: while its workgroups, two per compute unit, run in
-  // one round; larger batches run faster on the long-ring kernel)
+  // (a ring of chunks: while its workgroups, two per compute unit, run in one
+  // round. us a step of L=64 here and on the ring kernel, staggered fills and
+  // a lockstep cycle: B=8 (32 value heads) 7.2 and 7.6, 5.86 and 6.14; B=9 9.6
+  // and 8.3, 8.2 and 7.5; B=16 12.1 and 10.1, 9.0 and 8.0. The line could come
+  // down to one workgroup per compute unit: it is where it was against the
+  // replay kernel)
   return a.L <= gdnr::kDecodeChunks * gdnr::kStepRing && (a.V == 64 || a.V == 128) &&
          (int64_t)a.B * a.H * a.G <= 2 * (int64_t)gdnr::device_cus();
 }
@@ -575,9 +579,9 @@ int launch_ring(const gdnr::ReplayArgs& r, int act, bool fused, bool gate_f32, v
   // heads share their key head's staging, from three workgroups per compute
   // unit on (what is resident at once); four of 32 rows below that, where
   // twice the workgroups fill the chip and a flush is half as long. us per
-  // step with staggered fills, four and two waves: B=24, L=64 11.9 and 14.6;
-  // B=37, L=48 14.7 and 18.6; B=64, L=64 22.0 and 21.7; B=256 73 and 54
-  // (with the flushes whole).
+  // step with staggered fills, four and two waves: B=24, L=64 11.8 and 14.3;
+  // B=37, L=48 14.9 and 19.1; B=48, L=64 18.8 and 20.9; B=49 19.3 and 16.2;
+  // B=64 22.8 and 19.1; B=256 79.6 and 57.3.
   const int64_t resident = 3 * (int64_t)gdnr::device_cus();
   a.nwh = a.V == 256 || a.G % 2 || (a.V == 128 && (int64_t)a.B * a.H * (a.G / 2) <= resident) ? 4 : 2;
   a.gw = 4 / a.nwh;
@@ -1046,8 +1050,8 @@ int gdnr_prep_replay_fp8_slots(const gdnr_tensor* mixed_qkv, const gdnr_tensor* 
   // <= 64 with V <= 128 at small batches), else the ring kernel (16-bit
   // activations, rings of 17 to 64 tokens; both 64-bit slot bases, 32-bit
   // offsets inside a slot), else the step kernel (rings of <= 16 tokens,
-  // tensors under 2 GiB), else the long-ring kernel (rings of up to 64
-  // tokens, every address in 64 bits)
+  // tensors under 2 GiB), else the replay kernel (gdnr_kernels.hip: rings of
+  // up to 64 tokens, every address in 64 bits)
   if (decode_eligible(r, g.act) && decode_offsets_fit(r, elem_size(g.act))) {
     fit_decode(&r);
     return hip_status(launch_decode(r, g.act, true, a->dtype == GDNR_DTYPE_F32, stream));

@@ -16,7 +16,7 @@ namespace gdnr {
 namespace {
 
 constexpr int K = kKeyDim;
-constexpr int NT = kStepRing;  // token rows of the operands (ring capacity <= 16)
+constexpr int NT = kStepRing;  // token rows of an operand (a ring of up to 16 tokens, or a chunk of a longer one)
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));

@@ -2,8 +2,7 @@
 // gfx950: head, row, tile and vblock granularity, fp8 e4m3fn or int8 codes
 // (prototype/gdn_replay_fp8_reference.py:36-37,40-106 quantise, :109-134
 // dequantise), for a per-layer choice of format. The decode path itself
-// reads vblock/32 fp8 (gdnr_kernels.hip has the fast vblock32 quantiser);
-// these kernels build and read the other formats.
+// reads vblock/32 fp8; these kernels build and read that and the others.
 //
 // A scale group is the set of state elements that share one scale:
 //   head    rows [0, V)           x columns [0, K)

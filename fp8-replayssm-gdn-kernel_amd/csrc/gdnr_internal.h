@@ -74,8 +74,18 @@ struct ReplayArgs {
 constexpr int32_t kMaxStepLds = 160 * 1024;  // gfx950 LDS per workgroup
 constexpr int kStepRing = 16;                // ring capacity handled by the step kernel
 constexpr int kDecodeChunks = 4;             // chunks of kStepRing tokens of the decode kernel's longest ring
-constexpr int kRingOrder = 256;               // sequences the ring kernel orders (flushes first)
-constexpr int kRingHalves = 8;                // flushing sequences it gives two workgroups each
+// Sequences the ring kernel orders (flushes first). Finding the order costs
+// every workgroup its metadata's round trip: us a launch of L=64 in the batch's
+// order and ordered, with no, 8 and 64 flushes: B=256 50.5 and 56.6, 68.1 and
+// 62.5, 125 and 92; B=320 67.0 and 74.8, 82.4 and 80.8, 114 and 109; B=400 85.2
+// and 96.6, 100.0 and 103.5, 128.6 and 129.9. Staggered fills bring B / L
+// flushes a launch (4 to 6 here): the order pays for itself up to about B=300.
+constexpr int kRingOrder = 256;
+// Flushing sequences it gives two workgroups each, all of them or (past this
+// many) none: us a launch of B=64, L=64 with none, up to 8 and up to 16 in
+// halves: one flush 24.4, 21.6 and 21.6; four 25.1, 22.0 and 22.0; eight 26.0,
+// 26.2 and 26.2; twelve 26.3, 26.3 and 27.4; B=128 gains nothing with any.
+constexpr int kRingHalves = 8;
 constexpr uint32_t kWaitPolls = 1u << 22;     // default poll budget of a bounded LDS wait
 
 // Argument block of the step kernel (gdnr_step.hip), built on the host from a

@@ -13,12 +13,13 @@
 //   5. the checkpoint matvec o = (codes . T) * scale on the VALU (no MFMA:
 //      one FMA per byte), rows reduced across 8 lanes with DPP.
 // The order of steps 2-3 is pinned with compiler fences.
-// These kernels serve the split path, the standalone prep and the rings that the others leave: longer than 16 tokens with f32
-// activations (or a V the ring kernel does not hold, or tensors past its
-// 32-bit offsets). Rings of up to 16 tokens go through the decode kernel
-// (gdnr_decode.hip, 16-bit activations) or the step kernel (gdnr_step.hip,
-// f32 activations), longer ones of 16-bit activations through the decode
-// kernel (small batches) or the ring kernel (gdnr_ring.hip).
+// These kernels serve the split path, the standalone prep and the rings that
+// the others leave: longer than 16 tokens with f32 activations, a V the ring
+// kernel does not hold (V = 64 with an odd group, 32, 96, ...) or tensors past
+// its 32-bit offsets. Rings of up to 16 tokens go through the decode kernel
+// (gdnr_decode.hip, 16-bit activations) or the step kernel (gdnr_step.hip, f32
+// activations), longer ones of 16-bit activations through the decode kernel
+// (small batches) or the ring kernel (gdnr_ring.hip).
 //
 // This file is compiled once per activation dtype: GDNR_ACT=0 (bf16), 1
 // (f16), 2 (f32).

@@ -6,17 +6,20 @@
 // Workgroup: 4 waves of 32 VB V-rows = GW value heads of one key head and
 // sequence (WPH waves a head). No wave streams on its own: all four stage the
 // key ring, form the Gram matrix and stream checkpoint rows, and meet at three
-// barriers. Three workgroups share a compute unit (40 KiB of LDS, 168 VGPRs:
+// barriers. Three workgroups share a compute unit (40 KiB of LDS, 158 VGPRs:
 // held to 128, for four, the flush spills and every launch with one is slower,
 // B=64, L=64 20.3 to 31.6 us against 21.7), so one's serial part (the
 // coefficient chain) overlaps the others' streams.
 //
 // Bound: a replay at full batch by its bytes and its VALU issue (B=64, L=64,
-// fill 32: 60 MB in 17.4 us, 3.5 TB/s, against 25.3 for the per-token chain of
-// gdnr_kernels.hip that this kernel replaces; fill 63 22.1 against 36.0); a
+// fill 32: 60 MB in 19.0 us, 3.2 TB/s, against 25.8 for the per-token chain of
+// gdnr_kernels.hip that this kernel replaces; fill 63 23.9 against 36.9); a
 // flush by its waves' own latency (6 us to the factors, then 3.7 us a tile: a
-// launch of 24 flushes 25 us against 192). A step of B=64, L=64 with one
-// sequence flushing takes 18.0 us against 140.
+// launch of 24 flushes 26 us against 193). A step of B=64, L=64 with staggered
+// fills (one sequence flushing) takes 18.6 us against 134. Short fills gain
+// nothing, and where many rounds of small workgroups repeat the staging (V=64
+// or an odd group) they lose: B=200, L=17 at fill 8, 16 heads of V=64 17.1
+// against 14.1.
 //
 // Replay (the adjoint of the reference's reverse chain,
 // prototype/gdn_replayssm_fp8_kernel.py:121-173, in Gram form over the whole
@@ -80,7 +83,7 @@ constexpr int ring_lds(int gw, int vb) {
   const int replay = gw * (kT0Bytes + kCoefBytes) + NW * 32 * vb * 4, flush = gw * (kRBytes + kFacBytes + kLamBytes) + 2 * NW * 4;
   return kLdsZ + (replay > flush ? replay : flush);
 }
-static_assert(ring_lds(2, 2) <= 40 * 1024, "four workgroups share a compute unit's LDS");
+static_assert(ring_lds(2, 2) <= 40 * 1024, "a compute unit holds four workgroups' LDS (and three's registers)");
 
 typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
@@ -175,8 +178,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
   // round of workgroups (m_order: 1 + the grid's rows past the batch) takes
   // the flushing sequences first, and a few of them with two workgroups each:
   // a flush runs longer than a replay, and one that starts in the last round
-  // ends the launch late. B=64, L=64, one flush a step: 27.8 us in the batch's
-  // order, 21.1 flushes first, 18.0 in halves too (replays alone 17.4). The
+  // ends the launch late. B=64, L=64, one flush a step: 24.5 us in the batch's
+  // order, 22.0 flushes first, 18.6 in halves too (replays alone, at fill 32,
+  // 18.5 in the batch's order and 19.0 with the order looked for). The
   // blockIdx.y-th sequence of that order is found from every sequence's flag;
   // its lane holds its metadata too.
   int b = blockIdx.y, bs = b, n, pos = -1;
@@ -920,7 +924,7 @@ int launch_shape(const StepArgs& a, bool fused, bool gate_f32, hipStream_t s) {
 
 }  // namespace
 
-// a.nwh waves of a.V / a.nwh rows per value head (fit_ring)
+// a.nwh waves of a.V / a.nwh rows per value head (launch_ring in gdnr_abi.cpp)
 int GDNR_SUFFIX(launch_ring)(const StepArgs& a, bool fused, bool gate_f32, void* stream) {
   const hipStream_t s = (hipStream_t)stream;
   if (a.nwh == 2) return a.V == 128 ? launch_shape<2, 2>(a, fused, gate_f32, s) : launch_shape<1, 2>(a, fused, gate_f32, s);
