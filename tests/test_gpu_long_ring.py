@@ -124,11 +124,10 @@ def test_long_ring_fused_equals_prep_then_replay(device):
 
 
 def test_long_ring_tiles_identical(device):
-    """The V-tile height of the long-ring kernel (block_v 32, 64 or 128; the
-    library also lowers it on its own for small launches) changes nothing:
+    """The requested V-tile height (block_v 32, 64 or 128) changes nothing:
     outputs, requantised codes and scales are bit-identical at L = 64, with
-    replaying and flushing sequences in the same launch. (Batch 16: no tile
-    is lowered below the requested one.)"""
+    replaying and flushing sequences in the same launch. (Batch 16 of this
+    layer runs the decode kernel, which has no V-tiles.)"""
     from gpu_helpers import make_replay_case, run_replay
 
     valid = [64, 17, 33, 64, 1, 64, 50, 63, 64, 2, 40, 64, 9, 64, 31, 64]
@@ -203,3 +202,23 @@ def test_replay_kernel_16_bit(device, batch, heads, value_heads, value_dim, wind
         assert rel_l2(out[i], ref[i]) <= 2.0 ** -8, (i, valid[i], flush[i])
     assert np.mean(codes != ref_codes) < 1e-4
     assert np.abs(scale.view(np.int16).astype(np.int32) - ref_scale.view(np.int16).astype(np.int32)).max() <= 1
+
+
+@pytest.mark.parametrize("batch,heads,value_heads,value_dim,window,dtype,tiles", [
+    (43, 4, 12, 64, 40, torch.bfloat16, (64, 32)), (16, 16, 32, 128, 20, torch.float32, (64, 32))])
+def test_replay_kernel_tiles_identical(device, batch, heads, value_heads, value_dim, window, dtype, tiles):
+    """The replay kernel's V-tile height changes nothing, bit for bit, with
+    replaying and flushing sequences in the same launch. (Batches at which the
+    library lowers no tile below the requested one.)"""
+    from gpu_helpers import make_replay_case, run_replay
+
+    valid = np.array([(11 * i) % window + 1 for i in range(batch)])
+    flush = valid % 3 == 0
+    results = []
+    for tile in tiles:
+        case = make_replay_case(batch, window, device, seed=4500, heads=heads, value_heads=value_heads,
+                                value_dim=value_dim, dtype=dtype, warmup=8, valid=valid, flush=flush)
+        out = run_replay(case, block_v=tile)
+        results.append((out, case["ckpt"].payload.view(torch.uint8).clone(), case["ckpt"].scale.clone()))
+    for x, y in zip(*results):
+        assert torch.equal(x, y)

@@ -109,7 +109,7 @@ def test_slots_beyond_4096_equal_direct_path(device, L, nseq):
     sequence flushes): outputs, ring rows and checkpoint bytes equal the
     direct path's on batch-ordered copies, bit for bit. L = 8: the decode
     kernel; L = 64 (6.4 GiB of cache): its chunked path with 6 sequences,
-    the long-ring kernel with 17."""
+    the ring kernel with 17."""
     B, steps, n_slots = nseq, L + 2, 5000
     shape = synth.Shape(B)
     gen = synth.generator(63, device)
