@@ -88,6 +88,12 @@ int dtype_code(at::ScalarType t) {
   }
 }
 
+// the interpreter lock released for a scope (exceptions leave it held again)
+struct Unlocked {
+  PyThreadState* state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
 // C++ exceptions (torch's) become Python ones at every function's edge
 template <class Fn>
 PyObject* guarded(Fn&& fn) {
@@ -169,7 +175,12 @@ PyObject* host_empty(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       shape.push_back(PyLong_AsLongLong(PyTuple_GET_ITEM(args[1], i)));
       if (PyErr_Occurred()) return nullptr;
     }
-    return THPVariable_Wrap(at::empty(shape, at::TensorOptions().dtype(like.dtype()).device(like.device())));
+    const auto options = at::TensorOptions().dtype(like.dtype()).device(like.device());
+    // (an allocation may wait for the device, and that for another thread)
+    return THPVariable_Wrap([&] {
+      Unlocked unlocked;
+      return at::empty(shape, options);
+    }());
   });
 }
 
@@ -255,10 +266,12 @@ PyObject* host_call(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       stream = c10::hip::getCurrentHIPStream(device->index()).stream();
     }
     int status;
-    PyThreadState* state = PyEval_SaveThread();
-    status = e.sig->invoke(e.fn, ptr.data(), ints.data(), floats.data(), stream);
-    const std::string message = status ? g_last_error() : "";  // (thread-local in the library)
-    PyEval_RestoreThread(state);
+    std::string message;
+    {
+      Unlocked unlocked;
+      status = e.sig->invoke(e.fn, ptr.data(), ints.data(), floats.data(), stream);
+      if (status) message = g_last_error();  // (thread-local in the library)
+    }
     if (status == 0) Py_RETURN_NONE;
     PyObject* error = PyObject_CallFunction(g_error_class, "is", status, message.c_str());
     if (error) {

@@ -5,6 +5,9 @@ status as GdnrError)."""
 
 from __future__ import annotations
 
+import threading
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -138,3 +141,29 @@ def test_step_packs_on_the_host_under_any_default_device(host, monkeypatch):
     with torch.device("meta"):
         cache.step([3, 0], rows, rows, rows, rows[:0], rows[:0], q_out=rows)
     assert launch.pos.tolist() == [0, -1] and launch.valid.tolist() == [1, 0]
+
+
+def test_empty_lets_other_threads_run(host):
+    """An allocation may wait for the device, and what the device waits for may
+    need another thread: the interpreter lock is released meanwhile. (The
+    allocation made slow: torch fills new memory under its deterministic mode.)"""
+    like, ticks, stop = torch.empty(0, dtype=torch.bfloat16), [], threading.Event()
+
+    def tick():
+        while not stop.wait(0.001):
+            ticks.append(time.perf_counter())
+
+    thread = threading.Thread(target=tick)
+    thread.start()
+    torch.use_deterministic_algorithms(True)
+    try:
+        start = time.perf_counter()
+        made = host.empty(like, (1 << 26,))
+        end = time.perf_counter()
+    finally:
+        torch.use_deterministic_algorithms(False)
+        stop.set()
+        thread.join()
+    assert made.shape == (1 << 26,) and made.dtype == like.dtype
+    margin = 0.2 * (end - start)
+    assert any(start + margin < t < end - margin for t in ticks)
