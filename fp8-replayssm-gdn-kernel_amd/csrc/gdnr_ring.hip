@@ -738,39 +738,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
           q[cc] = qa + qb;
         }
       }
-      // A value that is infinite in the last token makes its row of the state
-      // +-inf (beta v k^T) in the recurrence, and the row's vblock is scaled
-      // by that; the products above make NaN of the whole row (0 inf, and inf
-      // - inf between U~'s parts). Such rows are found here and written after
-      // the product. (An infinity anywhere else in the ring, or a NaN, makes
-      // NaN of the row in the recurrence too.)
-      uint32_t inf_rows = 0, neg_rows = 0;  // bit l16
-      if (__builtin_expect(__any(!(__builtin_fabsf(o) < __builtin_inff())), 0)) {
-        bool rest = scp < __builtin_inff(), mine = false, neg = false;
-        auto finite = [](float x) { return __builtin_fabsf(x) < __builtin_inff(); };
-        // (v and the codes read again: the loop's registers are left alone)
-#pragma unroll 1
-        for (int k = 0; k < 4 * NF; ++k) {
-          const int t = NT * (k >> 2) + 4 * q4 + (k & 3);
-          if (t >= n) continue;
-          const uint8_t* vt = FUSED && t == pos ? f_new : f_rows + (uint32_t)t * a.v_t;
-          const float x = act_val(*(const uint16_t*)(vt + (32 * p + l16) * ES));
-          const float2 f = *(const float2*)(fl + 8 * t);
-          rest = rest && finite(f.x) && finite(f.y) && finite(*(const float*)(lds + kLdsDq + 4 * t));
-          if (t + 1 < n) rest = rest && finite(x);
-          else mine = __builtin_fabsf(x) == __builtin_inff() && f.y != 0.f, neg = (x < 0.f) != (f.y < 0.f);
-        }
-#pragma unroll 1
-        for (int k = 0; k < 8; ++k) {
-          const uint32_t w = ld32(fc_rows + (uint32_t)(32 * p + l16) * a.ck_v + 32 * q4 + 4 * k);
-          rest = rest && (((w & 0x7F7F7F7Fu) + 0x01010101u) & 0x80808080u) == 0;
-        }
-        // (the four lanes of a row)
-        uint64_t rm = __ballot(rest), im = __ballot(mine), nm = __ballot(mine && neg);
-        rm &= rm >> 32, im |= im >> 32, nm |= nm >> 32;
-        rm &= rm >> 16, im |= im >> 16, nm |= nm >> 16;
-        inf_rows = (uint32_t)(rm & im) & 0xFFFFu, neg_rows = (uint32_t)nm;
-      }
       // U~ decayed to the end of the ring, and the checkpoint's own weight
 #pragma unroll
       for (int c = 0; c < NF - 1; ++c) q[c] *= ll[4 + c];
@@ -838,13 +805,44 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
 #pragma unroll
         for (int ct = 0; ct < 8; ++ct) sv[ct] *= down;
       }
-      if (inf_rows) {
-        const float x = (neg_rows >> l16) & 1 ? -__builtin_inff() : __builtin_inff();
+      // A value that is infinite in the last token makes its row of the state
+      // +-inf (beta v k^T) in the recurrence, and the row's vblock is scaled
+      // by that; the products make NaN of the whole row (0 inf, and inf - inf
+      // between U~'s parts). Such rows are found and written here. (An infinity
+      // anywhere else in the ring, or a NaN, makes NaN of the row in the
+      // recurrence too.)
+      if (__builtin_expect(__any(!(__builtin_fabsf(o) < __builtin_inff())), 0)) {
+        bool rest = scp < __builtin_inff(), mine = false, neg = false;
+        auto finite = [](float x) { return __builtin_fabsf(x) < __builtin_inff(); };
+        // (v and the codes read again: the loop's registers are left alone)
+#pragma unroll 1
+        for (int k = 0; k < 4 * NF; ++k) {
+          const int t = NT * (k >> 2) + 4 * q4 + (k & 3);
+          if (t >= n) continue;
+          const uint8_t* vt = FUSED && t == pos ? f_new : f_rows + (uint32_t)t * a.v_t;
+          const float x = act_val(*(const uint16_t*)(vt + (32 * p + l16) * ES));
+          const float2 f = *(const float2*)(fl + 8 * t);
+          rest = rest && finite(f.x) && finite(f.y) && finite(*(const float*)(lds + kLdsDq + 4 * t));
+          if (t + 1 < n) rest = rest && finite(x);
+          else mine = __builtin_fabsf(x) == __builtin_inff() && f.y != 0.f, neg = (x < 0.f) != (f.y < 0.f);
+        }
+#pragma unroll 1
+        for (int k = 0; k < 8; ++k) {
+          const uint32_t w = ld32(fc_rows + (uint32_t)(32 * p + l16) * a.ck_v + 32 * q4 + 4 * k);
+          rest = rest && (((w & 0x7F7F7F7Fu) + 0x01010101u) & 0x80808080u) == 0;
+        }
+        // (the four lanes of a row)
+        uint64_t rm = __ballot(rest), im = __ballot(mine), nm = __ballot(mine && neg);
+        rm &= rm >> 32, im |= im >> 32, nm |= nm >> 32;
+        rm &= rm >> 16, im |= im >> 16, nm |= nm >> 16;
+        if (((rm & im) >> l16) & 1) {
+          const float x = (nm >> l16) & 1 ? -__builtin_inff() : __builtin_inff();
 #pragma unroll
-        for (int ct = 0; ct < 8; ++ct) {
-          const uint2 kw = *(const uint2*)(lds + kLdsX + (n - 1) * kXS + 64 * q4 + 8 * ct);
-          const float2 k01 = Act::from_pair(kw.x), k23 = Act::from_pair(kw.y);
-          if ((inf_rows >> l16) & 1) sv[ct] = f32x4_t{x * k01.x, x * k01.y, x * k23.x, x * k23.y};
+          for (int ct = 0; ct < 8; ++ct) {
+            const uint2 kw = *(const uint2*)(lds + kLdsX + (n - 1) * kXS + 64 * q4 + 8 * ct);
+            const float2 k01 = Act::from_pair(kw.x), k23 = Act::from_pair(kw.y);
+            sv[ct] = f32x4_t{x * k01.x, x * k01.y, x * k23.x, x * k23.y};
+          }
         }
       }
       // (the next vblock's codes, while this one is requantised)
