@@ -103,14 +103,13 @@ class ReplaySSMCache:
         """One full-contract decode step of the batch: batch entry i is the
         sequence in slot slots[i] (0 = padding; its output is meaningless).
         mixed_qkv [B, 2HK + HV V], a, b [B, HV]; returns out [B, HV, V]."""
-        slots = np.asarray(slots, dtype=np.int64)
-        if slots.ndim != 1:  # (ascontiguousarray makes a scalar a vector)
+        slots = np.asarray(slots, dtype=np.int64, order="C")
+        if slots.ndim != 1:
             raise ValueError("slots must be one-dimensional")
-        slots = np.ascontiguousarray(slots)
         host = gdnr_lib.host()
         # (the extension takes int64 fills; an array of another type that
         # replaced them steps on a copy)
-        fill = np.ascontiguousarray(self.fill, dtype=np.int64)
+        fill = np.asarray(self.fill, dtype=np.int64, order="C")
         batch = slots.shape[0]
         # slot, pos, valid_len (int32) and flush (a byte) of each entry, in one
         # pinned buffer and one copy
