@@ -6,7 +6,7 @@
 // Workgroup: 4 waves of 32 VB V-rows = GW value heads of one key head and
 // sequence (WPH waves a head). No wave streams on its own: all four stage the
 // key ring, form the Gram matrix and stream checkpoint rows, and meet at three
-// barriers. Three workgroups share a compute unit (40 KiB of LDS, 158 VGPRs:
+// barriers. Three workgroups share a compute unit (40 KiB of LDS, 155 VGPRs:
 // held to 128, for four, the flush spills and every launch with one is slower,
 // B=64, L=64 20.3 to 31.6 us against 21.7), so one's serial part (the
 // coefficient chain) overlaps the others' streams.
