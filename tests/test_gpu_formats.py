@@ -50,13 +50,22 @@ def test_format_matches_oracle(device, gran, tile):
 
 
 def test_vblock32_paths_agree(device):
-    """The decode path's fast vblock32 quantiser and the generic one write the same bytes."""
+    """The decode path's vblock32 entry point and the formats' one write the
+    same bytes, the latter on the stripe kernel and (rows whose stride is no
+    multiple of four elements) on the generic one; both read them back alike."""
+    import gdnr_lib
+
     x = _state(device, 71)
     fast = gk.quantize_checkpoint(x, "vblock", 32)
-    payload = torch.empty_like(fast.payload)
-    scale = torch.empty_like(fast.scale)
-    import gdnr_lib
-    gdnr_lib.call("gdnr_quantize_checkpoint", [x, payload, scale, None], [3, 32],
-                  gdnr_lib.current_stream(device))
-    assert torch.equal(payload.view(torch.uint8), fast.payload.view(torch.uint8))
-    assert torch.equal(scale, fast.scale)
+    back = gk.dequantize_checkpoint(fast)
+    odd = torch.empty(*x.shape[:3], 131, device=device)[..., :128]
+    for state in (x, odd.copy_(x)):
+        payload = torch.empty_like(fast.payload)
+        scale = torch.empty_like(fast.scale)
+        gdnr_lib.call("gdnr_quantize_checkpoint", [state, payload, scale, None], [3, 32],
+                      gdnr_lib.current_stream(device))
+        assert torch.equal(payload.view(torch.uint8), fast.payload.view(torch.uint8))
+        assert torch.equal(scale, fast.scale)
+        state.zero_()
+        gdnr_lib.call("gdnr_dequantize_checkpoint", [payload, scale, state], [3, 32], gdnr_lib.current_stream(device))
+        assert torch.equal(state.contiguous().view(torch.int32), back.view(torch.int32))
