@@ -82,3 +82,62 @@ def test_ring_kernel_edges(device, name):
     assert np.mean(codes[rows] != ref_codes) < 1e-4
     ulp = np.abs(scale[rows].view(np.int16).astype(np.int32) - ref_scale.view(np.int16).astype(np.int32))
     assert ulp.max() <= 1
+
+
+@pytest.mark.parametrize("batch", [20, 64])
+def test_ring_kernel_strided_views(device, batch):
+    """Operands at the loosest strides and alignments the entry point takes
+    (mixed_qkv rows that start 4 bytes past a 16-byte boundary, padded
+    checkpoint rows, ring rows and scales that are slices, index vectors with
+    gaps) give what contiguous copies give, bit for bit, and nothing beside
+    the views is written."""
+    heads, value_heads, value_dim, ring = 16, 32, 128, 40
+    valid = np.array([(9 * i) % ring + 1 for i in range(batch)])
+    flush = np.array([i % 4 == 1 for i in range(batch)])
+    case = make_replay_case(batch, ring, device, seed=11, warmup=4, valid=valid, flush=flush, reference_dist=True)
+    shape = synth.Shape(batch, heads, value_heads, value_dim=value_dim)
+    gen = synth.generator(12, device)
+    a_log, dt_bias = synth.gating_params(shape, gen, device, reference_dist=True)
+    mixed, a, b = (t[:, 0].contiguous() for t in synth.raw_step_inputs(shape, 1, gen, device))
+
+    def within(t, pads):
+        """A copy of t as a slice of a larger buffer: pads[d] = (before, after) of dim d."""
+        big = torch.full([n + lo + hi for n, (lo, hi) in zip(t.shape, pads)], 0x55, dtype=torch.uint8,
+                         device=device).to(t.dtype)
+        view = big[tuple(slice(lo, lo + n) for n, (lo, _) in zip(t.shape, pads))]
+        return big, view.copy_(t)
+
+    def gaps(t, step):
+        big = torch.zeros(step * t.shape[0], dtype=t.dtype, device=device)
+        return big[::step].copy_(t)
+
+    payload = case["ckpt"].payload.view(torch.uint8)
+    state = [payload, case["ckpt"].scale, case["k"], case["v"], case["g"], case["beta"]]
+    pads = [[(0, 0), (0, 1), (0, 0), (16, 48)], [(0, 0), (0, 0), (1, 2)], [(0, 0), (3, 1), (0, 0), (0, 8)],
+            [(0, 0), (0, 2), (0, 0), (8, 0)], [(0, 0), (1, 1), (1, 0)], [(1, 0), (0, 0), (3, 0)]]
+    pos = case["valid"] - 1
+    results = []
+    for strided in (False, True):
+        if strided:
+            bigs, views = zip(*(within(t, p) for t, p in zip(state, pads)))
+            out_big, out = within(torch.zeros(batch, value_heads, value_dim, dtype=mixed.dtype, device=device),
+                                  [(0, 0), (0, 0), (1, 2)])
+            q_big, q_out = within(torch.zeros_like(case["q"]), [(0, 0), (0, 1), (2, 4)])
+            m, aa, bb = within(mixed, [(0, 0), (2, 4)])[1], within(a, [(0, 0), (1, 2)])[1], within(b, [(1, 1), (0, 3)])[1]
+            index = [gaps(pos, 2), gaps(case["valid"], 3), gaps(case["flush"], 3)]
+        else:
+            views = [t.clone() for t in state]
+            out, q_out = torch.zeros(batch, value_heads, value_dim, dtype=mixed.dtype, device=device), torch.zeros_like(case["q"])
+            m, aa, bb, index = mixed, a, b, [pos, case["valid"], case["flush"]]
+        codes, scale, *rings = views
+        gk.gdn_prep_replay_fp8(m, aa, bb, a_log, dt_bias, index[0], codes.view(torch.float8_e4m3fn), scale, q_out, *rings,
+                               index[1], index[2], out=out)
+        results.append([out, q_out, *views])
+    assert (m.data_ptr() % 16, m.stride(0) * 2 % 16) == (4, 12)
+    for x, y in zip(*results):
+        assert torch.equal(x, y)
+    for big, t, p in [*zip(bigs, state, pads), (out_big, results[1][0], [(0, 0), (0, 0), (1, 2)]),
+                      (q_big, results[1][1], [(0, 0), (0, 1), (2, 4)])]:
+        inside = torch.zeros(big.shape, dtype=torch.bool, device=device)
+        inside[tuple(slice(lo, lo + n) for n, (lo, _) in zip(t.shape, p))] = True
+        assert bool((big[~inside] == torch.full((), 0x55, dtype=torch.uint8, device=device).to(big.dtype)).all())
